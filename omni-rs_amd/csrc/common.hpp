@@ -216,6 +216,9 @@ __device__ __forceinline__ void s_waitcnt_vm() {
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((LGKM0 ? 0 : 15) << 8) | ((N >> 4) << 14));
 }
 
+// s_waitcnt lgkmcnt(0): this wave's LDS operations are done.
+__device__ __forceinline__ void s_waitcnt_lgkm0() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // Workgroup barrier for the LDS-DMA pipeline. __syncthreads() would wait for
 // every outstanding vector-memory operation (its release fence counts the
 // in-flight global->LDS copies as LDS writes); here the caller has already

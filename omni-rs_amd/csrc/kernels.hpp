@@ -63,6 +63,9 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream);
 // current device (0: no split); with fewer in W8A8Args it splits less.
 int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width);
 hipError_t launch_w8a8_scalar(const W8A8Args& a, hipStream_t stream);
+// The weight-streaming kernel for up to 64 rows (rows.hip); no workspace.
+bool w8a8_rows_fits(const W8A8Args& a);
+hipError_t launch_w8a8_rows(const W8A8Args& a, hipStream_t stream);
 
 struct W8A16Args {
     const _Float16* x;      // [rows][width]

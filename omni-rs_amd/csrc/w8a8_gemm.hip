@@ -1507,6 +1507,7 @@ int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width) {
     a.columns = columns;
     a.width = width;
     if (!ring_offsets_fit(a)) return 0;
+    if (w8a8_tile_override() == 0 && w8a8_rows_fits(a)) return 0;  // no split there
     const int sp = w8a8_auto_splits(rows, columns, width, num_cus());
     return sp > 1 ? (int64_t)sp * rows * columns : 0;
 }
@@ -1526,6 +1527,15 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream) {
         case 16: return launch_pair<192>(a, stream);
         case 17: return launch_pair<128>(a, stream, w8a8_split_override());
         case 19: return launch_ring8_256(a, stream);
+        case 30:
+            if (w8a8_rows_fits(a)) return launch_w8a8_rows(a, stream);
+            break;
+        case 0:
+            // Up to 64 rows the weights' stream is all that counts: on every
+            // shape measured (rows.hip) the streaming kernel is ahead of the
+            // 256-row tiles below.
+            if (w8a8_rows_fits(a)) return launch_w8a8_rows(a, stream);
+            break;
         default: break;
     }
     // Cost model, fitted to MI355X timings of every candidate on ten shapes
