@@ -7,6 +7,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <atomic>
+#include <initializer_list>
 #include <mutex>
 
 #include "../../include/omni_int8.h"
@@ -110,6 +111,24 @@ std::atomic<int> g_cus[kMaxDevices];
 // unset, the measured rule below.
 int w8a16_route() { return omni::knob(omni::Knob::W8A16Route, 0); }
 
+// A knob that pins a kernel or a split keeps the call off the streaming
+// kernels (rows.hip), which have none of their own.
+bool pinned(std::initializer_list<omni::Knob> knobs) {
+    constexpr int kUnset = INT32_MIN;
+    for (omni::Knob k : knobs)
+        if (omni::knob(k, kUnset) != kUnset) return true;
+    return false;
+}
+bool w8a16_pinned() {
+    using K = omni::Knob;
+    return pinned({K::W8A16Route, K::W8A16Gemv, K::W8A16Skinny, K::W8A16SkinnySplit, K::W8A16Tile, K::W8A16Splits});
+}
+bool w4a16_pinned() {
+    using K = omni::Knob;
+    return pinned({K::W8A16Route, K::W4A16Gemv, K::W4A16SkinnySplit, K::W4A16Tile, K::W4A16Splits});
+}
+
+// Where the streaming kernels do not take the call (w8a16_rows_take):
 // 17..64 rows: the skinny kernel streams the weights once per 16 rows, the
 // GEMM once per 64 to 256, so the GEMM wins on big matrices (MI355X, W8A16
 // 4096 -> 14336: 24.5 against 37.7 us at 24 rows, 27.4 against 70.5 at 64;
@@ -127,8 +146,10 @@ bool midrows_take_gemm(int64_t rows, int64_t columns, int64_t width, bool int4, 
     return elems >= 32e6;
 }
 
-// The W8A16 route: 0 GEMV, 1 skinny MFMA, 2 the GEMM. `a` gives the shape
-// (and, for W4A16, the group and scale layout) the ring check reads.
+// The W8A16 route apart from the streaming kernels: 0 GEMV, 1 skinny MFMA, 2
+// the GEMM. `a` gives the shape (and, for W4A16, the group and scale layout)
+// the ring check reads. The workspace sizes follow it (a call that the
+// streaming kernels take leaves its workspace unused).
 int w8a16_kind(const omni::W8A16Args& a) {
     const int64_t rows = a.rows, columns = a.columns, width = a.width;
     // The GEMV spreads a row over one workgroup of at most 1024 lanes, one
@@ -234,6 +255,7 @@ int f16_linear(const char* name, const uint16_t* x, const uint16_t* w, int64_t r
     // The GEMV gives a row to one workgroup of at most 1024 lanes with up to
     // four 8-element chunks each: width <= 32768.
     if (rows <= 4 && width <= 32768) return hip_status(omni::launch_f16_gemv(a, s), "f16 gemv launch");
+    if (omni::f16_rows_take(a)) return hip_status(omni::launch_f16_rows(a, s), "f16 rows launch");
     if (rows <= 64) return hip_status(omni::launch_f16_skinny(a, s), "f16 skinny launch");
     return hip_status(omni::launch_f16_mfma(a, s), "f16 mfma launch");
 }
@@ -626,6 +648,8 @@ int omni_w8a16_gemm_ws(const uint16_t* x, const int8_t* w, const uint16_t* scale
     a.partial = static_cast<float*>(workspace);
     a.partial_elems = (int64_t)(workspace_bytes / sizeof(float));
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (!w8a16_pinned() && omni::w8a16_rows_take(a))
+        return hip_status(omni::launch_w8a16_rows(a, s), "w8a16 rows launch");
     switch (w8a16_kind(a)) {
         case 0: return hip_status(omni::launch_w8a16_gemv(a, s), "w8a16 gemv launch");
         case 1: return hip_status(omni::launch_w8a16_skinny(a, s), "w8a16 skinny launch");
@@ -685,6 +709,8 @@ int omni_w4a16_gemm_ws(const uint16_t* x, const uint8_t* w_packed, const uint16_
     a.partial = static_cast<float*>(workspace);
     a.partial_elems = (int64_t)(workspace_bytes / sizeof(float));
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (!w4a16_pinned() && omni::w4a16_rows_take(a))
+        return hip_status(omni::launch_w4a16_rows(a, s), "w4a16 rows launch");
     switch (w4a16_kind(a)) {
         case 0: return hip_status(omni::launch_w4a16_gemv(a, s), "w4a16 gemv launch");
         case 1: return hip_status(omni::launch_w4a16_skinny(a, s), "w4a16 skinny launch");

@@ -86,6 +86,15 @@ struct W8A16Args {
 bool w8a16_ring_usable(const W8A16Args& a);
 bool w4a16_ring_usable(const W8A16Args& a);
 
+// The weight-streaming kernels for up to 64 rows (rows.hip), and whether they
+// are this call's best route; no workspace.
+bool w8a16_rows_take(const W8A16Args& a);
+bool w4a16_rows_take(const W8A16Args& a);
+bool f16_rows_take(const W8A16Args& a);
+hipError_t launch_w8a16_rows(const W8A16Args& a, hipStream_t stream);
+hipError_t launch_w4a16_rows(const W8A16Args& a, hipStream_t stream);
+hipError_t launch_f16_rows(const W8A16Args& a, hipStream_t stream);
+
 hipError_t launch_w8a16_gemv(const W8A16Args& a, hipStream_t stream);
 hipError_t launch_w8a16_skinny(const W8A16Args& a, hipStream_t stream);
 hipError_t launch_w8a16_mfma(const W8A16Args& a, hipStream_t stream);

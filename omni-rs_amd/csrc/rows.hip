@@ -1,5 +1,6 @@
-// Linears of up to 64 rows on gfx950, bound by the stream of their weights
-// (columns x width bytes; the matrix cores need a fraction of its time).
+// Linears of up to 64 rows on gfx950 (W8A8, and int8, int4 or f16 weights
+// under f16 activations), bound by the stream of their weights; the matrix
+// cores need a fraction of its time.
 //
 // A workgroup of KW waves walks blocks of 16 NB columns (units), each wave a
 // KW-th of K, in tiles of TB bytes of K. Everything a tile needs, 16 NB
@@ -22,33 +23,44 @@
 // 4096 x 28672 23.4 against 40.3, 14336 x 4096 13.3 against 26.3 (the bare
 // read: 4.0, 5.4, 18.5, 10.4); 48 rows of 4096 x 6144 11.0 against 28.2;
 // 8 rows of 4304 x 1152 (K % 64 != 0) 5.6 against 48.
+#include <type_traits>
+
 #include "common.hpp"
+#include "dequant.hpp"
 #include "kernels.hpp"
 
 namespace omni {
 
 namespace {
 
-// The weights' kind. W8A8's activations are int8 codes.
-enum : int { kW8A8 = 0 };
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
-template <int WK>
-struct Kind {
-    static constexpr int kXBytes = 1;   // activation bytes per weight byte
-    using Acc = v4i;
-};
+// The weights' kind: int8 under int8 activation codes (exact int32 sums),
+// int8, packed int4 (group 128) and f16 under f16 activations.
+enum : int { kW8A8, kW8A16, kW4A16, kF16 };
+
+// Activation bytes per weight byte.
+constexpr int x_bytes(int wk) { return wk == kW8A16 ? 2 : wk == kW4A16 ? 4 : 1; }
+
+constexpr int kInt4Group = 128;
 
 struct RowsArgs {
-    const uint8_t* x;   // [rows][width] codes
-    const uint8_t* w;   // [columns][width]
-    int64_t rows, columns, width;
-    // The epilogue, as in W8A8Args.
+    const uint8_t* x;   // [rows][width], codes or f16
+    const uint8_t* w;   // [columns][row_bytes]
+    int64_t rows, columns;
+    int row_bytes;      // of a weight row
+    void* out;
+    // The f16 epilogue: scale (W8A16) and bias per column, either may be null;
+    // int4's group scales, bf16 [columns][width / 128].
+    const _Float16* scale16;
+    const _Float16* bias16;
+    const uint16_t* gscale;
+    // The W8A8 epilogue, as in W8A8Args.
     const float* x_scale;
     const int32_t* x_sum;
     const float* w_scale;
     const int32_t* w_zero;
     const float* bias;
-    void* out;
     int32_t* acc_dump;
     bool out_f16;
 };
@@ -85,24 +97,27 @@ constexpr int kStreamColumns = 512;
 // never stored).
 template <int WK, int MB, int NB, int XC, int S, int KW, int TB>
 __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a) {
-    using Kd = Kind<WK>;
-    using Acc = typename Kd::Acc;
-    constexpr int XTB = TB * Kd::kXBytes;        // activation bytes per row and tile
+    using Acc = std::conditional_t<WK == kW8A8, v4i, v4f>;
+    using Sum = std::conditional_t<WK == kW8A8, int, float>;
+    constexpr int XTB = TB * x_bytes(WK);        // activation bytes per row and tile
     constexpr int RPC = 1024 / TB, XR = 1024 / XTB;  // rows per copy
     constexpr int BN = 16 * NB;
-    constexpr int WC = BN / RPC, C = WC + XC;    // copies per tile
+    constexpr int WC = BN / RPC;                 // weight copies per tile
+    constexpr int SC = WK == kW4A16 ? 1 : 0;     // group scale copies (4 bytes per lane)
+    constexpr int C = WC + XC + SC;
     constexpr int XROWS = XC * XR;               // activation rows held
     static_assert(XROWS == 16 * MB || (MB == 1 && XROWS < 16 && (XROWS & (XROWS - 1)) == 0), "activation rows");
-    constexpr int kStage = C * 1024;
+    static_assert(WK != kW4A16 || (TB == kInt4Group && BN <= 64), "one dword of group scales per column and tile");
+    constexpr int kStage = (WC + XC) * 1024 + SC * 256;
     constexpr int kSteps = TB / 64;
     constexpr int T = 64 * KW;
     constexpr int kPart = MB * NB * 256;         // partial sums per wave
     __shared__ __attribute__((aligned(1024))) uint8_t stages[KW * S * kStage];
-    __shared__ int part[KW * kPart];
+    __shared__ Sum part[KW * kPart];
     __shared__ float s_scale[16 * MB];
     __shared__ int s_sum[16 * MB];
     __shared__ float s_ws[kStreamColumns];
-    __shared__ int s_zero[kStreamColumns];
+    __shared__ int s_zero[WK == kW8A8 ? kStreamColumns : 1];
     __shared__ float s_bias[kStreamColumns];
 
     const int tid = threadIdx.x;
@@ -112,7 +127,7 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
     const int units = (int)((a.columns + BN - 1) / BN);
     const int first = blockIdx.x, stride = gridDim.x;
     const int nu = (units - first + stride - 1) / stride;  // units of this workgroup (first < units)
-    const int wrow = (int)a.width;
+    const int wrow = a.row_bytes;
     const int ktiles = (wrow + TB - 1) / TB;
     const int lo = wave * ktiles / KW, mine = (wave + 1) * ktiles / KW - lo;
     const bool tail = wrow % TB != 0;
@@ -134,9 +149,11 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
     for (int c = 0; c < XC; ++c) {
         const int r = c * XR + lane / (XTB / 16);
         xch[c] = ((lane % (XTB / 16)) ^ ((r / kXW) & kXMask)) * 16;
-        xoff[c] = (unsigned)(min((int64_t)r, a.rows - 1) * wrow * Kd::kXBytes);
+        xoff[c] = (unsigned)(min((int64_t)r, a.rows - 1) * wrow * x_bytes(WK));
     }
     const unsigned st_lds = lds_addr(stages) + wave * (S * kStage);
+    // int4: bytes of a column's group scales (one group per 64 weight bytes).
+    const int srow = wrow / 64 * 2;
     auto issue = [&](int unit, int tile, int slot) {
         const int64_t n0 = (int64_t)(first + unit * stride) * BN;
         const uint8_t* wb = a.w + n0 * wrow;
@@ -147,9 +164,13 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
             const unsigned off = (unsigned)(min(wrow_l[c], cols - 1) * wrow + min(tile * TB + wch[c], wrow - 16));
             lds_copy16_nt(off, wb, dst + c * 1024);
         }
+        if constexpr (SC != 0) {
+            const unsigned off = (unsigned)(min(lane, cols - 1) * srow + tile * 4);
+            lds_copy4_saddr(off, reinterpret_cast<const uint8_t*>(a.gscale) + n0 * srow, dst + (WC + XC) * 1024);
+        }
 #pragma unroll
         for (int c = 0; c < XC; ++c) {
-            const unsigned off = xoff[c] + (unsigned)min(tile * XTB + xch[c], wrow * Kd::kXBytes - 16);
+            const unsigned off = xoff[c] + (unsigned)min(tile * XTB + xch[c], wrow * x_bytes(WK) - 16);
             lds_copy16_saddr(off, a.x, dst + (WC + c) * 1024);
         }
     };
@@ -165,16 +186,23 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
         if (s < total) issue_next(s);
 
     const bool has_zero = a.w_zero != nullptr, has_bias = a.bias != nullptr;
-    for (int i = tid; i < 16 * MB; i += T) {
-        const int64_t row = min((int64_t)i, a.rows - 1);
-        s_scale[i] = a.x_scale[row];
-        s_sum[i] = has_zero ? a.x_sum[row] : 0;
+    if constexpr (WK == kW8A8) {
+        for (int i = tid; i < 16 * MB; i += T) {
+            const int64_t row = min((int64_t)i, a.rows - 1);
+            s_scale[i] = a.x_scale[row];
+            s_sum[i] = has_zero ? a.x_sum[row] : 0;
+        }
     }
     for (int i = tid; i < nu * BN; i += T) {
         const int64_t n = min((int64_t)(first + i / BN * stride) * BN + i % BN, a.columns - 1);
-        s_ws[i] = a.w_scale[n];
-        s_zero[i] = has_zero ? a.w_zero[n] : 0;
-        s_bias[i] = has_bias ? a.bias[n] : -0.0f;  // x + -0.0 is x
+        if constexpr (WK == kW8A8) {
+            s_ws[i] = a.w_scale[n];
+            s_zero[i] = has_zero ? a.w_zero[n] : 0;
+            s_bias[i] = has_bias ? a.bias[n] : -0.0f;  // x + -0.0 is x
+        } else {
+            s_ws[i] = a.scale16 ? (float)a.scale16[n] : 1.0f;
+            s_bias[i] = a.bias16 ? (float)a.bias16[n] : 0.0f;
+        }
     }
 
     const int wkey = (r16 / kW) & kWMask;
@@ -189,33 +217,74 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
             for (int i = 0; i < MB; ++i) acc[j][i] = Acc{};
         for (int t = 0; t < mine; ++t) {
             wait_tiles<C, S>(issued - done - 1);
-            const uint8_t* ws = stages + (wave * S + slot) * kStage + r16 * TB;
-            const uint8_t* xs = stages + (wave * S + slot) * kStage + WC * 1024 + xr * XTB;
-            v4i b[kSteps][NB], x[kSteps][MB];
+            const uint8_t* st = stages + (wave * S + slot) * kStage;
+            const uint8_t* ws = st + r16 * TB;
+            const uint8_t* xs = st + WC * 1024 + xr * XTB;
+            const bool last = tail && lo + t == ktiles - 1;
 #pragma unroll
             for (int s = 0; s < kSteps; ++s) {
+                // Lane (r, g) holds weight bytes 64 s + 16 g .. +15 of column r's
+                // tile (16 int8 codes, 32 int4 codes, 8 halves), and the
+                // activations of row r at the same k. Past the row's end both
+                // are zero.
+                const bool out_of_row = last && (lo + t) * TB + s * 64 + g * 16 >= wrow;
+                v4u w[NB];
 #pragma unroll
-                for (int j = 0; j < NB; ++j)
-                    b[s][j] = *reinterpret_cast<const v4i*>(ws + j * 16 * TB + (((4 * s + g) ^ wkey) << 4));
+                for (int j = 0; j < NB; ++j) {
+                    w[j] = *reinterpret_cast<const v4u*>(ws + j * 16 * TB + (((4 * s + g) ^ wkey) << 4));
+                    if (last && out_of_row) w[j] = v4u{0u, 0u, 0u, 0u};
+                }
+                if constexpr (WK == kW8A8) {
 #pragma unroll
-                for (int i = 0; i < MB; ++i)
-                    x[s][i] = *reinterpret_cast<const v4i*>(xs + i * 16 * XTB + (((4 * s + g) ^ xkey) << 4));
-            }
-            if (tail && lo + t == ktiles - 1) {
+                    for (int i = 0; i < MB; ++i) {
+                        const v4i x = *reinterpret_cast<const v4i*>(xs + i * 16 * XTB + (((4 * s + g) ^ xkey) << 4));
 #pragma unroll
-                for (int s = 0; s < kSteps; ++s)
-                    if ((lo + t) * TB + s * 64 + g * 16 >= wrow) {
-#pragma unroll
-                        for (int j = 0; j < NB; ++j) b[s][j] = v4i{0, 0, 0, 0};
+                        for (int j = 0; j < NB; ++j)
+                            acc[j][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, __builtin_bit_cast(v4i, w[j]),
+                                                                             acc[j][i], 0, 0, 0);
                     }
+                } else {
+                    constexpr int kH = x_bytes(WK);  // 8-code halves of the lane's codes
+                    v8h b[NB][kH];
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) {
+                        v2h h[4 * kH];
+                        if constexpr (WK == kF16) {
+                            __builtin_memcpy(h, &w[j], 16);
+                        } else if constexpr (WK == kW8A16) {
+                            i8x4_to_f16x4(w[j].x, h[0], h[1]);
+                            i8x4_to_f16x4(w[j].y, h[2], h[3]);
+                            i8x4_to_f16x4(w[j].z, h[4], h[5]);
+                            i8x4_to_f16x4(w[j].w, h[6], h[7]);
+                        } else {
+                            const u32 two = *reinterpret_cast<const u32*>(st + (WC + XC) * 1024 + (j * 16 + r16) * 4);
+                            const float sf = bf16_to_f32((uint16_t)(s == 0 ? two & 0xffffu : two >> 16));
+                            const _Float16 sc = last && out_of_row ? (_Float16)0.0f : (_Float16)sf;
+                            v2h lo8[8], hi8[8];
+                            i4x16_dequant(w[j].x, w[j].y, sc, lo8);
+                            i4x16_dequant(w[j].z, w[j].w, sc, hi8);
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) h[e] = lo8[e], h[8 + e] = hi8[e];
+                        }
+#pragma unroll
+                        for (int q = 0; q < kH; ++q)
+                            b[j][q] = v8h{h[4 * q][0],     h[4 * q][1],     h[4 * q + 1][0], h[4 * q + 1][1],
+                                          h[4 * q + 2][0], h[4 * q + 2][1], h[4 * q + 3][0], h[4 * q + 3][1]};
+                    }
+#pragma unroll
+                    for (int q = 0; q < kH; ++q) {
+                        const int chunk = 4 * kH * s + kH * g + q;
+#pragma unroll
+                        for (int i = 0; i < MB; ++i) {
+                            v8h x = *reinterpret_cast<const v8h*>(xs + i * 16 * XTB + ((chunk ^ xkey) << 4));
+                            if (last && out_of_row) x = v8h{};
+#pragma unroll
+                            for (int j = 0; j < NB; ++j)
+                                acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, b[j][q], acc[j][i], 0, 0, 0);
+                        }
+                    }
+                }
             }
-#pragma unroll
-            for (int s = 0; s < kSteps; ++s)
-#pragma unroll
-                for (int j = 0; j < NB; ++j)
-#pragma unroll
-                    for (int i = 0; i < MB; ++i)
-                        acc[j][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[s][i], b[s][j], acc[j][i], 0, 0, 0);
             if (issued < total) {
                 s_waitcnt_lgkm0();  // the slot is read
                 issue_next(slot);
@@ -239,22 +308,31 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
             const int row = e / BN, col = u * BN + e % BN;
             const int64_t n = (int64_t)(first + u * stride) * BN + e % BN;
             if (e < kPart && row < a.rows && n < a.columns) {
-                unsigned sum = 0;
-#pragma unroll
-                for (int k = 0; k < KW; ++k) sum += (unsigned)part[k * kPart + e];
                 const int64_t idx = row * a.columns + n;
-                if (a.acc_dump) a.acc_dump[idx] = (int)sum;
-                float o;
-                {
+                if constexpr (WK == kW8A8) {
+                    unsigned sum = 0;
+#pragma unroll
+                    for (int k = 0; k < KW; ++k) sum += (unsigned)part[k * kPart + e];
+                    if (a.acc_dump) a.acc_dump[idx] = (int)sum;
+                    float o;
+                    {
+                        // crates/omni-kernel/src/int8_matmul.rs:156-158: wrapping
+                        // int32, then two multiplies and the bias, each rounded.
 #pragma clang fp contract(off)
-                    const int centered = (int)(sum - (unsigned)s_sum[row] * (unsigned)s_zero[col]);
-                    const float t = (float)centered * s_scale[row];
-                    o = t * s_ws[col] + s_bias[col];
+                        const int centered = (int)(sum - (unsigned)s_sum[row] * (unsigned)s_zero[col]);
+                        const float t = (float)centered * s_scale[row];
+                        o = t * s_ws[col] + s_bias[col];
+                    }
+                    if (a.out_f16)
+                        static_cast<_Float16*>(a.out)[idx] = (_Float16)o;
+                    else
+                        static_cast<float*>(a.out)[idx] = o;
+                } else {
+                    float sum = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < KW; ++k) sum += part[k * kPart + e];
+                    static_cast<_Float16*>(a.out)[idx] = (_Float16)(sum * s_ws[col] + s_bias[col]);
                 }
-                if (a.out_f16)
-                    static_cast<_Float16*>(a.out)[idx] = (_Float16)o;
-                else
-                    static_cast<float*>(a.out)[idx] = o;
             }
         }
         s_waitcnt_lgkm0();  // before the next unit's barrier
@@ -277,41 +355,193 @@ hipError_t launch_stream_cfg(const RowsArgs& a, int64_t cus, hipStream_t stream)
 
 }  // namespace
 
-// Byte offsets are 32-bit within 32 weight rows and within the activations.
-bool w8a8_rows_fits(const W8A8Args& a) {
-    return a.rows <= 64 && a.width % 16 == 0 && a.width >= 16 && a.width <= 131072;
+namespace {
+
+// Blocks of 16 columns outnumber the CUs.
+bool is_wide(int64_t columns, int64_t cus) { return columns > 16 * cus; }
+
+// One activation byte per weight byte (W8A8, f16 weights). Measured over K x
+// N of 1152 ... 14336 x 1152 ... 28672 at 1 to 64 rows of W8A8. Where one block
+// of 16 columns per CU covers the matrix, eight waves share it (from 17 rows
+// on the rings leave LDS for four). On wider matrices up to 8 rows take two
+// four-wave workgroups per CU (8 rows of 4096 x 6144 7.9 against 8.4 us, of
+// 4096 x 28672 23.1 against 24.0), more rows blocks of 32 columns, which
+// halve the activations' share of the copies (48 rows of 4096 x 6144 11.0
+// against 13.9 us, of 4096 x 28672 36.0 against 43).
+template <int WK>
+hipError_t launch_even(const RowsArgs& a, hipStream_t st) {
+    const int64_t cus = num_cus();
+    const bool wide = is_wide(a.columns, cus);
+    if (a.rows <= 4)
+        return wide ? launch_stream_cfg<WK, 1, 1, 1, 2, 4, 256>(a, cus, st)
+                    : launch_stream_cfg<WK, 1, 1, 1, 3, 8, 256>(a, cus, st);
+    if (a.rows <= 8)
+        return wide ? launch_stream_cfg<WK, 1, 1, 2, 2, 4, 256>(a, cus, st)
+                    : launch_stream_cfg<WK, 1, 1, 2, 2, 8, 256>(a, cus, st);
+    if (a.rows <= 16)
+        return wide ? launch_stream_cfg<WK, 1, 2, 2, 2, 8, 128>(a, cus, st)
+                    : launch_stream_cfg<WK, 1, 1, 4, 2, 8, 256>(a, cus, st);
+    if (a.rows <= 32)
+        return wide ? launch_stream_cfg<WK, 2, 2, 4, 3, 4, 128>(a, cus, st)
+                    : launch_stream_cfg<WK, 2, 1, 8, 2, 4, 256>(a, cus, st);
+    if (a.rows <= 48)
+        return wide ? launch_stream_cfg<WK, 3, 2, 6, 3, 4, 128>(a, cus, st)
+                    : launch_stream_cfg<WK, 3, 1, 6, 3, 4, 128>(a, cus, st);
+    return wide ? launch_stream_cfg<WK, 4, 2, 8, 2, 4, 128>(a, cus, st)
+                : launch_stream_cfg<WK, 4, 1, 8, 2, 4, 128>(a, cus, st);
 }
 
-// Measured over K x N of 1152 ... 14336 x 1152 ... 28672 at 1 to 64 rows. Where
-// one block of 16 columns per CU covers the matrix, eight waves share it
-// (16 rows and fewer; the rings of more rows leave LDS for four). On wider
-// matrices up to 8 rows take two four-wave workgroups per CU (8 rows of 4096
-// x 6144 7.9 against 8.4 us, of 4096 x 28672 23.1 against 24.0), more rows
-// blocks of 32 columns, which halve the activations' share of the copies (48
-// rows of 4096 x 6144 11.0 against 13.9 us, of 4096 x 28672 36.0 against 43).
+RowsArgs f16_args(const W8A16Args& w, int64_t row_bytes) {
+    RowsArgs a{};
+    a.x = reinterpret_cast<const uint8_t*>(w.x);
+    a.w = reinterpret_cast<const uint8_t*>(w.w);
+    a.rows = w.rows;
+    a.columns = w.columns;
+    a.row_bytes = (int)row_bytes;
+    a.out = w.out;
+    a.scale16 = w.scale;
+    a.bias16 = w.bias;
+    a.gscale = w.gscale;
+    return a;
+}
+
+// Byte offsets are 32-bit within 64 weight rows and within the activations.
+constexpr int64_t kMaxRowBytes = 1 << 18;
+
+}  // namespace
+
+bool w8a8_rows_fits(const W8A8Args& a) {
+    return a.rows <= 64 && a.width % 16 == 0 && a.width >= 16 && a.width <= kMaxRowBytes;
+}
+
 hipError_t launch_w8a8_rows(const W8A8Args& w, hipStream_t st) {
     if (w.rows == 0 || w.columns == 0) return hipSuccess;
-    RowsArgs a{w.x,       w.w,      w.rows, w.columns, w.width,    w.x_scale, w.x_sum,
-               w.w_scale, w.w_zero, w.bias, w.out,     w.acc_dump, w.out_f16};
+    RowsArgs a{};
+    a.x = w.x;
+    a.w = w.w;
+    a.rows = w.rows;
+    a.columns = w.columns;
+    a.row_bytes = (int)w.width;
+    a.out = w.out;
+    a.x_scale = w.x_scale;
+    a.x_sum = w.x_sum;
+    a.w_scale = w.w_scale;
+    a.w_zero = w.w_zero;
+    a.bias = w.bias;
+    a.acc_dump = w.acc_dump;
+    a.out_f16 = w.out_f16;
+    return launch_even<kW8A8>(a, st);
+}
+
+// Five to 64 rows, against the skinny kernels and the GEMM (w8a16.hip):
+// 8 rows of 14336 x 4096 14.0 against 19.9 us, 16 of 4096 x 14336 16.5
+// against 21.3, 32 of 1536 x 17920 14.5 against 25.4, 48 of 8960 x 1536 18.7
+// against 29.7; one and two rows of K > 16384 (the GEMV's limit) 15.4 against
+// 21.4 (18944 x 3584). The others keep:
+//  * up to 16 rows at K = 1024, 2048, 3072, 4096 in one round of workgroups,
+//    the LDS skinny kernel built for that K (16 of 4096 x 4096 6.9 against
+//    7.5 us, of 1024 x 4096 3.4 against 3.8);
+//  * three and four rows, the GEMV up to K = 4096 on up to 8192 columns (4 of
+//    4096 x 4096 5.8 against 6.1, 3 of 5120 x 5120 9.0 against 9.4) and at K =
+//    4096 up to 64 M weights (4 of 4096 x 14336 13.9 against 14.5; beyond, 4
+//    of 4096 x 28672 22.8 against 24.1, of 14336 x 4096 12.6 against 15.3);
+//  * from 33 rows on, the GEMM where the matrix is large: each activation
+//    copy is then read by too few columns (48 of 4096 x 14336 28.3 against
+//    25.8 us, but of 4096 x 6144 15.1 against 29.2, of 14336 x 4096 29.9
+//    against 32.8; 64 of 2048 x 14336 18.6 against 17.4, of 4096 x 5120 15.7
+//    against 17.5, of 8960 x 1536 24.4 against 37.1).
+bool w8a16_rows_take(const W8A16Args& a) {
+    if (a.rows > 64 || a.width % 16 != 0 || a.width < 16 || a.width > kMaxRowBytes) return false;
+    const bool wide = is_wide(a.columns, num_cus());
+    const double elems = (double)a.columns * (double)a.width;
+    if (a.width > 16384 && a.rows <= 4) return true;
+    if (a.rows <= 2) return false;
+    if (a.rows <= 4) {
+        if (a.width == 4096 && elems <= (64 << 20)) return false;
+        return wide ? a.columns >= 8192 : a.width > 4096;
+    }
+    if (a.rows <= 16) return wide || a.width > 4096 || a.width % 1024 != 0;
+    if (a.rows <= 32) return true;
+    if (a.rows <= 48) return !wide || elems <= 36e6;
+    return elems < 16e6 || (a.width <= 4096 && elems <= 26e6);
+}
+
+hipError_t launch_w8a16_rows(const W8A16Args& w, hipStream_t st) {
+    if (w.rows == 0 || w.columns == 0) return hipSuccess;
+    const RowsArgs a = f16_args(w, w.width);
     const int64_t cus = num_cus();
-    const bool wide = w.columns > 16 * cus;
+    const bool wide = is_wide(a.columns, cus);
+    // Wide: two four-wave workgroups per CU, or from K = 4096 and 9 rows on
+    // blocks of 32 columns (8 rows of 4096 x 6144 7.7 against 8.8 us, of 1536
+    // x 17920 9.7 against 8.7; 16 rows of 4096 x 14336 16.5 against 21.4).
     if (w.rows <= 4)
-        return wide ? launch_stream_cfg<kW8A8, 1, 1, 1, 2, 4, 256>(a, cus, st)
-                    : launch_stream_cfg<kW8A8, 1, 1, 1, 3, 8, 256>(a, cus, st);
-    if (w.rows <= 8)
-        return wide ? launch_stream_cfg<kW8A8, 1, 1, 2, 2, 4, 256>(a, cus, st)
-                    : launch_stream_cfg<kW8A8, 1, 1, 2, 2, 8, 256>(a, cus, st);
+        return wide ? launch_stream_cfg<kW8A16, 1, 1, 2, 2, 4, 256>(a, cus, st)
+                    : launch_stream_cfg<kW8A16, 1, 1, 1, 3, 8, 128>(a, cus, st);
+    if (w.rows <= 8) {
+        if (!wide) return launch_stream_cfg<kW8A16, 1, 1, 2, 3, 8, 128>(a, cus, st);
+        return w.width >= 4096 ? launch_stream_cfg<kW8A16, 1, 2, 2, 2, 8, 128>(a, cus, st)
+                               : launch_stream_cfg<kW8A16, 1, 1, 2, 3, 4, 128>(a, cus, st);
+    }
     if (w.rows <= 16)
-        return wide ? launch_stream_cfg<kW8A8, 1, 2, 2, 2, 8, 128>(a, cus, st)
-                    : launch_stream_cfg<kW8A8, 1, 1, 4, 2, 8, 256>(a, cus, st);
+        return wide ? launch_stream_cfg<kW8A16, 1, 2, 4, 2, 8, 128>(a, cus, st)
+                    : launch_stream_cfg<kW8A16, 1, 1, 4, 3, 8, 128>(a, cus, st);
     if (w.rows <= 32)
-        return wide ? launch_stream_cfg<kW8A8, 2, 2, 4, 3, 4, 128>(a, cus, st)
-                    : launch_stream_cfg<kW8A8, 2, 1, 8, 2, 4, 256>(a, cus, st);
+        return wide ? launch_stream_cfg<kW8A16, 2, 2, 8, 2, 4, 128>(a, cus, st)
+                    : launch_stream_cfg<kW8A16, 2, 1, 8, 3, 4, 128>(a, cus, st);
     if (w.rows <= 48)
-        return wide ? launch_stream_cfg<kW8A8, 3, 2, 6, 3, 4, 128>(a, cus, st)
-                    : launch_stream_cfg<kW8A8, 3, 1, 6, 3, 4, 128>(a, cus, st);
-    return wide ? launch_stream_cfg<kW8A8, 4, 2, 8, 2, 4, 128>(a, cus, st)
-                : launch_stream_cfg<kW8A8, 4, 1, 8, 2, 4, 128>(a, cus, st);
+        return wide ? launch_stream_cfg<kW8A16, 3, 2, 6, 3, 4, 64>(a, cus, st)
+                    : launch_stream_cfg<kW8A16, 3, 1, 12, 2, 4, 128>(a, cus, st);
+    return wide ? launch_stream_cfg<kW8A16, 4, 2, 8, 2, 4, 64>(a, cus, st)
+                : launch_stream_cfg<kW8A16, 4, 1, 8, 3, 4, 64>(a, cus, st);
+}
+
+// Groups of 128, their scales copied two at a time: an even number per
+// column, on a 4-byte boundary. Three to 32 rows, against the GEMV and the
+// skinny kernels: 4 rows of 4096 x 6144 6.8 against 8.7 us, of 3584 x 18944
+// 13.2 against 15.9, 8 of 4096 x 14336 12.2 against 21.6, 16 of 14336 x 4096
+// 16.2 against 28.9, 32 of 3584 x 18944 29.8 against 40.3. The GEMV keeps
+// three and four rows of narrow long-K matrices (4 of 8960 x 1536 7.4
+// against 7.8); one and two rows of K > 32768 are past its limit.
+bool w4a16_rows_take(const W8A16Args& a) {
+    if (a.rows > 32 || a.group != kInt4Group || a.width % (2 * kInt4Group) != 0 || a.width <= 0 || a.width > kMaxRowBytes ||
+        reinterpret_cast<uintptr_t>(a.gscale) % 4 != 0)
+        return false;
+    if (a.width > 32768 && a.rows <= 4) return true;
+    if (a.rows <= 2) return false;
+    return a.rows > 4 || a.columns > 2048 || a.width <= 4096;
+}
+
+hipError_t launch_w4a16_rows(const W8A16Args& w, hipStream_t st) {
+    if (w.rows == 0 || w.columns == 0) return hipSuccess;
+    const RowsArgs a = f16_args(w, w.width / 2);
+    const int64_t cus = num_cus();
+    const bool wide = is_wide(a.columns, cus);
+    // Wide: blocks of 32 columns; up to 4 rows only where they still make a
+    // few rounds of long K (4096 x 6144 6.8 against 7.5 us, of 1536 x 17920
+    // 8.6 against 7.4).
+    if (w.rows <= 4) {
+        if (!wide) return launch_stream_cfg<kW4A16, 1, 1, 2, 3, 8, 128>(a, cus, st);
+        return w.width >= 4096 && w.columns <= 16384 ? launch_stream_cfg<kW4A16, 1, 2, 2, 2, 8, 128>(a, cus, st)
+                                                     : launch_stream_cfg<kW4A16, 1, 1, 2, 3, 4, 128>(a, cus, st);
+    }
+    if (w.rows <= 8)
+        return wide ? launch_stream_cfg<kW4A16, 1, 2, 4, 2, 8, 128>(a, cus, st)
+                    : launch_stream_cfg<kW4A16, 1, 1, 4, 2, 8, 128>(a, cus, st);
+    if (w.rows <= 16)
+        return wide ? launch_stream_cfg<kW4A16, 1, 2, 8, 2, 4, 128>(a, cus, st)
+                    : launch_stream_cfg<kW4A16, 1, 1, 8, 3, 4, 128>(a, cus, st);
+    return wide ? launch_stream_cfg<kW4A16, 2, 2, 16, 1, 4, 128>(a, cus, st)
+                : launch_stream_cfg<kW4A16, 2, 1, 16, 1, 4, 128>(a, cus, st);
+}
+
+// Five to 64 rows of f16 weights (up to 4 take the GEMV).
+bool f16_rows_take(const W8A16Args& a) {
+    return a.rows > 4 && a.rows <= 64 && a.width % 8 == 0 && a.width >= 8 && 2 * a.width <= kMaxRowBytes;
+}
+
+hipError_t launch_f16_rows(const W8A16Args& w, hipStream_t st) {
+    if (w.rows == 0 || w.columns == 0) return hipSuccess;
+    return launch_even<kF16>(f16_args(w, 2 * w.width), st);
 }
 
 }  // namespace omni

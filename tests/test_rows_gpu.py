@@ -5,6 +5,8 @@ import pytest
 import torch
 
 import omni_int8 as oi
+import tolerance
+from omni_int8 import f16
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +50,58 @@ def test_w8a8_stream_bit_exact(oracle, rows, width, columns):
         got = oi.w8a8_gemm(dev(codes), dev(rs), t, dev(w), dev(scale), z, dev(bias), torch.float16)
         _, o16 = oracle.w8a8_finish(acc, total, rs, scale, zero, bias)
         assert np.array_equal(host(got).view(np.uint16), o16)
+
+
+def close(got, want):
+    # f32 sums of products exact in f32 (W4A16: of weights rounded to f16, as
+    # the reference's own route rounds them), then one rounding to f16
+    assert tolerance.rel_err(host(got), want) <= tolerance.FP16_REL_TOL
+
+
+# Shapes that the streaming kernels take by default (w8a16_rows_take): every
+# row block, K % 64 and K % 256 not 0, one block and several per workgroup.
+@pytest.mark.parametrize("rows,width,columns", [
+    (1, 18944, 40), (4, 16400, 33), (3, 4112, 17), (4, 1552, 8195), (5, 16, 7), (6, 1040, 100), (8, 4624, 4100),
+    (8, 1168, 4112), (9, 4112, 64), (16, 240, 31), (13, 4096, 4113), (16, 528, 9000), (17, 64, 16), (32, 1104, 50),
+    (31, 336, 4130), (33, 272, 40), (48, 1040, 300), (47, 368, 4100), (49, 144, 30), (64, 2064, 70), (63, 400, 4101),
+    (24, 32, 131200)])
+def test_w8a16_stream(rows, width, columns):
+    rng = np.random.default_rng(rows + 3 * width + columns)
+    x = rng.standard_normal((rows, width)).astype(np.float16)
+    w = rng.integers(-128, 128, (columns, width), dtype=np.int8)
+    scale = rng.uniform(0.002, 0.02, columns).astype(np.float16)
+    bias = rng.standard_normal(columns).astype(np.float16)
+    exact = (x.astype(np.float64) @ w.T.astype(np.float64)) * scale.astype(np.float64)
+    close(oi.w8a16_linear(dev(x), dev(w), dev(scale)), exact)
+    close(oi.w8a16_linear(dev(x), dev(w), dev(scale), dev(bias)), exact + bias.astype(np.float64))
+    # a row's infinity stays in its row
+    x[0, width - 1] = np.inf
+    got = host(oi.w8a16_linear(dev(x), dev(w), dev(scale)))
+    assert not np.isfinite(got[0]).any() or (w[:, -1] == 0).any()
+    assert np.isfinite(got[1:]).all()
+
+
+@pytest.mark.parametrize("rows,width,columns", [
+    (1, 33024, 20), (3, 256, 5), (4, 2304, 33), (4, 4352, 2050), (3, 4352, 4100), (4, 512, 4100), (4, 256, 20000),
+    (5, 256, 15), (8, 1792, 100), (7, 768, 4100), (9, 3328, 17), (16, 256, 64), (13, 1280, 4097), (17, 512, 31),
+    (32, 2816, 70), (29, 768, 4129), (6, 256, 131100)])
+def test_w4a16_stream(oracle, rows, width, columns):
+    rng = np.random.default_rng(rows + 5 * width + columns)
+    x = rng.standard_normal((rows, width)).astype(np.float16)
+    packed = rng.integers(0, 256, (columns, width // 2), dtype=np.uint8)
+    scale = torch.from_numpy(rng.uniform(0.002, 0.02, (columns, width // 128)).astype(np.float32)).bfloat16()
+    bias = rng.standard_normal(columns).astype(np.float16)
+    q = np.stack((packed & 15, packed >> 4), -1).reshape(columns, width).astype(np.float64) - 8
+    exact = x.astype(np.float64) @ (q * np.repeat(scale.double().numpy(), 128, 1)).T
+    close(oi.w4a16_linear(dev(x), dev(packed), scale.cuda()), exact)
+    close(oi.w4a16_linear(dev(x), dev(packed), scale.cuda(), dev(bias)), exact + bias.astype(np.float64))
+
+
+@pytest.mark.parametrize("rows,width,columns", [
+    (5, 32, 9), (8, 160, 100), (9, 1056, 33), (16, 8192, 17), (17, 96, 64), (32, 544, 40), (33, 64, 31),
+    (48, 1120, 70), (49, 32, 16), (64, 2080, 95)])
+def test_f16_stream(rows, width, columns):
+    rng = np.random.default_rng(rows + width + columns)
+    x = rng.standard_normal((rows, width)).astype(np.float16)
+    w = (rng.standard_normal((columns, width)) * 0.05).astype(np.float16)
+    close(f16.depth_try_linear(dev(x), dev(w).t()), x.astype(np.float64) @ w.T.astype(np.float64))
