@@ -115,8 +115,8 @@ int omni_w8a8_gemm(const int32_t* x_packed, const float* x_scale, const int32_t*
                    const float* bias, int64_t rows, int64_t columns, int64_t width, void* out,
                    int out_dtype, int32_t* acc_dump, int lowering, void* stream);
 
-/* Bytes of workspace omni_w8a8_gemm_ws uses for this shape on the current
- * device: split-K partial sums (int32 [splits][rows][columns]) for shapes
+/* Bytes of workspace omni_w8a8_gemm_ws uses at most for this shape on the
+ * current device (a call of few rows may run without): split-K partial sums (int32 [splits][rows][columns]) for shapes
  * whose 256 x 128 output tiles alone would leave most CUs idle (the
  * reference's own 256-row benchmark shapes); 0 when the shape does not
  * split. */

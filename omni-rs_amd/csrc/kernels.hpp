@@ -63,9 +63,11 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream);
 // current device (0: no split); with fewer in W8A8Args it splits less.
 int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width);
 hipError_t launch_w8a8_scalar(const W8A8Args& a, hipStream_t stream);
-// The weight-streaming kernel for up to 64 rows (rows.hip); no workspace.
+// The weight-streaming kernels for few rows (rows.hip); no workspace. Above 64
+// rows: their estimated time in us, and the column blocks (2 or 4) it is for.
 bool w8a8_rows_fits(const W8A8Args& a);
-hipError_t launch_w8a8_rows(const W8A8Args& a, hipStream_t stream);
+double w8a8_rows_us(int64_t rows, int64_t columns, int64_t width, int* nb);
+hipError_t launch_w8a8_rows(const W8A8Args& a, int nb, hipStream_t stream);
 
 struct W8A16Args {
     const _Float16* x;      // [rows][width]
@@ -86,8 +88,8 @@ struct W8A16Args {
 bool w8a16_ring_usable(const W8A16Args& a);
 bool w4a16_ring_usable(const W8A16Args& a);
 
-// The weight-streaming kernels for up to 64 rows (rows.hip), and whether they
-// are this call's best route; no workspace.
+// The weight-streaming kernels for few rows (rows.hip), and whether they are
+// this call's best route; no workspace.
 bool w8a16_rows_take(const W8A16Args& a);
 bool w4a16_rows_take(const W8A16Args& a);
 bool f16_rows_take(const W8A16Args& a);

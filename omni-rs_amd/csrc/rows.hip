@@ -1,6 +1,8 @@
-// Linears of up to 64 rows on gfx950 (W8A8, and int8, int4 or f16 weights
-// under f16 activations), bound by the stream of their weights; the matrix
-// cores need a fraction of its time.
+// Linears of a few rows on gfx950 (W8A8, and int8, int4 or f16 weights under
+// f16 activations), bound by the stream of their weights; the matrix cores
+// need a fraction of its time. Up to 64 rows one workgroup sees them all;
+// more (small matrices, where 256-row tiles would leave most CUs idle) are cut
+// into tiles of 48 or 64.
 //
 // A workgroup of KW waves walks blocks of 16 NB columns (units), each wave a
 // KW-th of K, in tiles of TB bytes of K. Everything a tile needs, 16 NB
@@ -22,7 +24,10 @@
 // K x N = 4096 x 4096 6.1 against 14.3 us, 4096 x 6144 7.8 against 27.7,
 // 4096 x 28672 23.4 against 40.3, 14336 x 4096 13.3 against 26.3 (the bare
 // read: 4.0, 5.4, 18.5, 10.4); 48 rows of 4096 x 6144 11.0 against 28.2;
-// 8 rows of 4304 x 1152 (K % 64 != 0) 5.6 against 48.
+// 8 rows of 4304 x 1152 (K % 64 != 0) 5.6 against 48. In tiles: 128 rows of
+// 4096 x 4096 11.9 against 20.4 us, 256 rows 15.5 against 23.7 (split K), of
+// 3072 x 3072 13.5 against 33.6; a tile's K loop is bound by the copies into
+// LDS, 64 KiB per wave-tile step in 1.06 us per CU.
 #include <type_traits>
 
 #include "common.hpp"
@@ -89,112 +94,138 @@ __device__ __forceinline__ void wait_tiles(int tiles) {
     asm volatile("" ::: "memory");  // no LDS read moves above the wait
 }
 
-// Columns per workgroup, at most (their epilogue values are kept in LDS).
-constexpr int kStreamColumns = 512;
+// Units per workgroup, at most (their epilogue values are kept in LDS).
+constexpr int stream_units(int nb, bool mt) { return mt ? 8 : 32 / nb; }
 
 // XC activation copies per tile hold XC * XR rows: 16 MB, or for MB = 1 a
 // smaller power of two (the other rows of the block repeat them; they are
 // never stored).
-template <int WK, int MB, int NB, int XC, int S, int KW, int TB>
+template <int WK, int MB, int NB, int XC, int S, int KW, int TB, bool MT>
 __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a) {
     using Acc = std::conditional_t<WK == kW8A8, v4i, v4f>;
     using Sum = std::conditional_t<WK == kW8A8, int, float>;
     constexpr int XTB = TB * x_bytes(WK);        // activation bytes per row and tile
     constexpr int RPC = 1024 / TB, XR = 1024 / XTB;  // rows per copy
-    constexpr int BN = 16 * NB;
+    constexpr int BM = 16 * MB, BN = 16 * NB;
     constexpr int WC = BN / RPC;                 // weight copies per tile
     constexpr int SC = WK == kW4A16 ? 1 : 0;     // group scale copies (4 bytes per lane)
     constexpr int C = WC + XC + SC;
     constexpr int XROWS = XC * XR;               // activation rows held
-    static_assert(XROWS == 16 * MB || (MB == 1 && XROWS < 16 && (XROWS & (XROWS - 1)) == 0), "activation rows");
+    static_assert(XROWS == BM || (MB == 1 && !MT && XROWS < 16 && (XROWS & (XROWS - 1)) == 0), "activation rows");
     static_assert(WK != kW4A16 || (TB == kInt4Group && BN <= 64), "one dword of group scales per column and tile");
     constexpr int kStage = (WC + XC) * 1024 + SC * 256;
     constexpr int kSteps = TB / 64;
+    constexpr int kH = WK == kW8A8 ? 1 : x_bytes(WK);  // 16-byte activation pieces per lane and step
     constexpr int T = 64 * KW;
-    constexpr int kPart = MB * NB * 256;         // partial sums per wave
+    constexpr int NU = stream_units(NB, MT);
+    // Column blocks whose partial sums are added at a time.
+    constexpr int PJ = KW * MB * NB <= 32 ? NB : 1;
+    constexpr int PN = 16 * PJ, kPart = BM * PN;  // partial sums per wave
     __shared__ __attribute__((aligned(1024))) uint8_t stages[KW * S * kStage];
     __shared__ Sum part[KW * kPart];
-    __shared__ float s_scale[16 * MB];
-    __shared__ int s_sum[16 * MB];
-    __shared__ float s_ws[kStreamColumns];
-    __shared__ int s_zero[WK == kW8A8 ? kStreamColumns : 1];
-    __shared__ float s_bias[kStreamColumns];
+    __shared__ float s_scale[WK == kW8A8 ? (MT ? NU : 1) * BM : 1];
+    __shared__ int s_sum[WK == kW8A8 ? (MT ? NU : 1) * BM : 1];
+    __shared__ float s_ws[NU * BN];
+    __shared__ int s_zero[WK == kW8A8 ? NU * BN : 1];
+    __shared__ float s_bias[NU * BN];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
-    const int units = (int)((a.columns + BN - 1) / BN);
-    const int first = blockIdx.x, stride = gridDim.x;
+    const int tiles_m = MT ? (int)((a.rows + BM - 1) / BM) : 1;
+    const int units = (int)((a.columns + BN - 1) / BN) * tiles_m;
+    // Units of one column block are neighbours, and neighbours share an XCD,
+    // whose L2 then serves all but the first read of the weights.
+    const int first = MT ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x, stride = gridDim.x;
     const int nu = (units - first + stride - 1) / stride;  // units of this workgroup (first < units)
-    const int wrow = a.row_bytes;
+    const int wrow = a.row_bytes, xrow = wrow * x_bytes(WK);
     const int ktiles = (wrow + TB - 1) / TB;
     const int lo = wave * ktiles / KW, mine = (wave + 1) * ktiles / KW - lo;
     const bool tail = wrow % TB != 0;
+    auto unit_m0 = [&](int u) -> int64_t { return MT ? (int64_t)((first + u * stride) % tiles_m) * BM : 0; };
+    auto unit_n0 = [&](int u) -> int64_t { return (int64_t)(MT ? (first + u * stride) / tiles_m : first + u * stride) * BN; };
 
     // 16-byte chunk slots are XOR-swizzled by the row's 256-byte window, on
     // the global side of the copies.
     constexpr int kW = 256 / TB > 0 ? 256 / TB : 1;    // rows per 256-byte window
     constexpr int kXW = 256 / XTB > 0 ? 256 / XTB : 1;
     constexpr int kWMask = (TB / 16 - 1) & 15, kXMask = (XTB / 16 - 1) & 15;
-    int wrow_l[WC], wch[WC];
-    unsigned xoff[XC];
-    int xch[XC];
-#pragma unroll
-    for (int c = 0; c < WC; ++c) {
-        wrow_l[c] = c * RPC + lane / (TB / 16);
-        wch[c] = ((lane % (TB / 16)) ^ ((wrow_l[c] / kW) & kWMask)) * 16;
-    }
-#pragma unroll
-    for (int c = 0; c < XC; ++c) {
-        const int r = c * XR + lane / (XTB / 16);
-        xch[c] = ((lane % (XTB / 16)) ^ ((r / kXW) & kXMask)) * 16;
-        xoff[c] = (unsigned)(min((int64_t)r, a.rows - 1) * wrow * x_bytes(WK));
-    }
-    const unsigned st_lds = lds_addr(stages) + wave * (S * kStage);
+    auto w_row = [&](int c) { return c * RPC + lane / (TB / 16); };
+    auto w_byte = [&](int c) { return ((lane % (TB / 16)) ^ ((w_row(c) / kW) & kWMask)) * 16; };
+    auto x_row = [&](int c) { return c * XR + lane / (XTB / 16); };
+    auto x_byte = [&](int c) { return ((lane % (XTB / 16)) ^ ((x_row(c) / kXW) & kXMask)) * 16; };
     // int4: bytes of a column's group scales (one group per 64 weight bytes).
     const int srow = wrow / 64 * 2;
-    auto issue = [&](int unit, int tile, int slot) {
-        const int64_t n0 = (int64_t)(first + unit * stride) * BN;
-        const uint8_t* wb = a.w + n0 * wrow;
-        const int cols = (int)min((int64_t)BN, a.columns - n0);
+    // The copies' sources in the unit being issued: wave-uniform bases and
+    // per-lane offsets (rows past the matrix repeat the last one).
+    const uint8_t *wbase = nullptr, *xbase = a.x, *sbase = nullptr;
+    unsigned woff[WC], xoff[XC], soff = 0;
+    auto set_unit = [&](int u) {
+        const int64_t n0 = unit_n0(u), m0 = unit_m0(u);
+        const int cols = (int)min((int64_t)BN, a.columns - n0) - 1;
+        const int rows = (int)min((int64_t)BM, a.rows - m0) - 1;
+        wbase = a.w + n0 * wrow;
+        xbase = a.x + m0 * xrow;
+#pragma unroll
+        for (int c = 0; c < WC; ++c) woff[c] = (unsigned)(min(w_row(c), cols) * wrow + w_byte(c));
+#pragma unroll
+        for (int c = 0; c < XC; ++c) xoff[c] = (unsigned)(min(x_row(c), rows) * xrow + x_byte(c));
+        if constexpr (SC != 0) {
+            sbase = reinterpret_cast<const uint8_t*>(a.gscale) + n0 * srow;
+            soff = (unsigned)(min(lane, cols) * srow);
+        }
+    };
+    const unsigned st_lds = lds_addr(stages) + wave * (S * kStage);
+    auto issue = [&](int tile, int slot) {
         const unsigned dst = st_lds + slot * kStage;
+        const uint8_t* wb = wbase + tile * TB;
+        const uint8_t* xb = xbase + tile * XTB;
+        // A partial last tile: pieces past the row's end repeat its last one.
+        const bool last = tail && tile == ktiles - 1;
+        const int wend = wrow - 16 - tile * TB, xend = xrow - 16 - tile * XTB;
 #pragma unroll
         for (int c = 0; c < WC; ++c) {
-            const unsigned off = (unsigned)(min(wrow_l[c], cols - 1) * wrow + min(tile * TB + wch[c], wrow - 16));
-            lds_copy16_nt(off, wb, dst + c * 1024);
+            unsigned off = woff[c];
+            if (last) off -= max(w_byte(c) - wend, 0);
+            if constexpr (MT)
+                lds_copy16_saddr(off, wb, dst + c * 1024);
+            else
+                lds_copy16_nt(off, wb, dst + c * 1024);
         }
-        if constexpr (SC != 0) {
-            const unsigned off = (unsigned)(min(lane, cols - 1) * srow + tile * 4);
-            lds_copy4_saddr(off, reinterpret_cast<const uint8_t*>(a.gscale) + n0 * srow, dst + (WC + XC) * 1024);
-        }
+        if constexpr (SC != 0) lds_copy4_saddr(soff, sbase + tile * 4, dst + (WC + XC) * 1024);
 #pragma unroll
         for (int c = 0; c < XC; ++c) {
-            const unsigned off = xoff[c] + (unsigned)min(tile * XTB + xch[c], wrow * x_bytes(WK) - 16);
-            lds_copy16_saddr(off, a.x, dst + (WC + c) * 1024);
+            unsigned off = xoff[c];
+            if (last) off -= max(x_byte(c) - xend, 0);
+            lds_copy16_saddr(off, xb, dst + (WC + c) * 1024);
         }
     };
     const int total = mine * nu;
     int iu = 0, it = 0, issued = 0;  // next tile to issue
     auto issue_next = [&](int slot) {
-        issue(iu, lo + it, slot);
-        if (++it == mine) it = 0, ++iu;
+        issue(lo + it, slot);
         ++issued;
+        if (++it == mine) {
+            it = 0;
+            if (++iu < nu) set_unit(iu);
+        }
     };
+    set_unit(0);
 #pragma unroll
     for (int s = 0; s < S; ++s)
         if (s < total) issue_next(s);
 
     const bool has_zero = a.w_zero != nullptr, has_bias = a.bias != nullptr;
     if constexpr (WK == kW8A8) {
-        for (int i = tid; i < 16 * MB; i += T) {
-            const int64_t row = min((int64_t)i, a.rows - 1);
+        for (int i = tid; i < (MT ? nu : 1) * BM; i += T) {
+            const int64_t row = min(unit_m0(i / BM) + i % BM, a.rows - 1);
             s_scale[i] = a.x_scale[row];
             s_sum[i] = has_zero ? a.x_sum[row] : 0;
         }
     }
     for (int i = tid; i < nu * BN; i += T) {
-        const int64_t n = min((int64_t)(first + i / BN * stride) * BN + i % BN, a.columns - 1);
+        const int64_t n = min(unit_n0(i / BN) + i % BN, a.columns - 1);
         if constexpr (WK == kW8A8) {
             s_ws[i] = a.w_scale[n];
             s_zero[i] = has_zero ? a.w_zero[n] : 0;
@@ -220,49 +251,76 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
             const uint8_t* st = stages + (wave * S + slot) * kStage;
             const uint8_t* ws = st + r16 * TB;
             const uint8_t* xs = st + WC * 1024 + xr * XTB;
-            const bool last = tail && lo + t == ktiles - 1;
+            // Lane (r, g) holds weight bytes 64 s + 16 g .. +15 of column r's tile
+            // (16 int8 codes, 32 int4 codes, 8 halves), and the activations of
+            // row r at the same k.
+            v4u w[kSteps][NB], x[kSteps][MB][kH];
+            u32 sc2[NB];
 #pragma unroll
             for (int s = 0; s < kSteps; ++s) {
-                // Lane (r, g) holds weight bytes 64 s + 16 g .. +15 of column r's
-                // tile (16 int8 codes, 32 int4 codes, 8 halves), and the
-                // activations of row r at the same k. Past the row's end both
-                // are zero.
-                const bool out_of_row = last && (lo + t) * TB + s * 64 + g * 16 >= wrow;
-                v4u w[NB];
 #pragma unroll
-                for (int j = 0; j < NB; ++j) {
-                    w[j] = *reinterpret_cast<const v4u*>(ws + j * 16 * TB + (((4 * s + g) ^ wkey) << 4));
-                    if (last && out_of_row) w[j] = v4u{0u, 0u, 0u, 0u};
-                }
+                for (int j = 0; j < NB; ++j)
+                    w[s][j] = *reinterpret_cast<const v4u*>(ws + j * 16 * TB + (((4 * s + g) ^ wkey) << 4));
+#pragma unroll
+                for (int i = 0; i < MB; ++i)
+#pragma unroll
+                    for (int q = 0; q < kH; ++q)
+                        x[s][i][q] = *reinterpret_cast<const v4u*>(
+                            xs + i * 16 * XTB + (((4 * kH * s + kH * g + q) ^ xkey) << 4));
+            }
+            if constexpr (SC != 0) {
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    sc2[j] = *reinterpret_cast<const u32*>(st + (WC + XC) * 1024 + (j * 16 + r16) * 4);
+            }
+            // Everything is read: the slot takes the next tile while this one
+            // is multiplied.
+            if (issued < total) {
+                s_waitcnt_lgkm0();
+                issue_next(slot);
+            }
+            if (tail && lo + t == ktiles - 1) {
+                // Past the row's end both operands are zero (an infinity times
+                // a zero weight would not be).
+#pragma unroll
+                for (int s = 0; s < kSteps; ++s)
+                    if ((lo + t) * TB + s * 64 + g * 16 >= wrow) {
+#pragma unroll
+                        for (int j = 0; j < NB; ++j) w[s][j] = v4u{0u, 0u, 0u, 0u};
+#pragma unroll
+                        for (int i = 0; i < MB; ++i)
+#pragma unroll
+                            for (int q = 0; q < kH; ++q) x[s][i][q] = v4u{0u, 0u, 0u, 0u};
+                    }
+            }
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) {
                 if constexpr (WK == kW8A8) {
 #pragma unroll
-                    for (int i = 0; i < MB; ++i) {
-                        const v4i x = *reinterpret_cast<const v4i*>(xs + i * 16 * XTB + (((4 * s + g) ^ xkey) << 4));
+                    for (int i = 0; i < MB; ++i)
 #pragma unroll
                         for (int j = 0; j < NB; ++j)
-                            acc[j][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, __builtin_bit_cast(v4i, w[j]),
+                            acc[j][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, x[s][i][0]),
+                                                                             __builtin_bit_cast(v4i, w[s][j]),
                                                                              acc[j][i], 0, 0, 0);
-                    }
                 } else {
-                    constexpr int kH = x_bytes(WK);  // 8-code halves of the lane's codes
                     v8h b[NB][kH];
 #pragma unroll
                     for (int j = 0; j < NB; ++j) {
+                        const v4u wq = w[s][j];
                         v2h h[4 * kH];
                         if constexpr (WK == kF16) {
-                            __builtin_memcpy(h, &w[j], 16);
+                            __builtin_memcpy(h, &wq, 16);
                         } else if constexpr (WK == kW8A16) {
-                            i8x4_to_f16x4(w[j].x, h[0], h[1]);
-                            i8x4_to_f16x4(w[j].y, h[2], h[3]);
-                            i8x4_to_f16x4(w[j].z, h[4], h[5]);
-                            i8x4_to_f16x4(w[j].w, h[6], h[7]);
+                            i8x4_to_f16x4(wq.x, h[0], h[1]);
+                            i8x4_to_f16x4(wq.y, h[2], h[3]);
+                            i8x4_to_f16x4(wq.z, h[4], h[5]);
+                            i8x4_to_f16x4(wq.w, h[6], h[7]);
                         } else {
-                            const u32 two = *reinterpret_cast<const u32*>(st + (WC + XC) * 1024 + (j * 16 + r16) * 4);
-                            const float sf = bf16_to_f32((uint16_t)(s == 0 ? two & 0xffffu : two >> 16));
-                            const _Float16 sc = last && out_of_row ? (_Float16)0.0f : (_Float16)sf;
+                            const _Float16 sc = (_Float16)bf16_to_f32((uint16_t)(s == 0 ? sc2[j] & 0xffffu : sc2[j] >> 16));
                             v2h lo8[8], hi8[8];
-                            i4x16_dequant(w[j].x, w[j].y, sc, lo8);
-                            i4x16_dequant(w[j].z, w[j].w, sc, hi8);
+                            i4x16_dequant(wq.x, wq.y, sc, lo8);
+                            i4x16_dequant(wq.z, wq.w, sc, hi8);
 #pragma unroll
                             for (int e = 0; e < 8; ++e) h[e] = lo8[e], h[8 + e] = hi8[e];
                         }
@@ -272,90 +330,86 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
                                           h[4 * q + 2][0], h[4 * q + 2][1], h[4 * q + 3][0], h[4 * q + 3][1]};
                     }
 #pragma unroll
-                    for (int q = 0; q < kH; ++q) {
-                        const int chunk = 4 * kH * s + kH * g + q;
+                    for (int q = 0; q < kH; ++q)
 #pragma unroll
-                        for (int i = 0; i < MB; ++i) {
-                            v8h x = *reinterpret_cast<const v8h*>(xs + i * 16 * XTB + ((chunk ^ xkey) << 4));
-                            if (last && out_of_row) x = v8h{};
+                        for (int i = 0; i < MB; ++i)
 #pragma unroll
                             for (int j = 0; j < NB; ++j)
-                                acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, b[j][q], acc[j][i], 0, 0, 0);
-                        }
-                    }
+                                acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, x[s][i][q]),
+                                                                                  b[j][q], acc[j][i], 0, 0, 0);
                 }
-            }
-            if (issued < total) {
-                s_waitcnt_lgkm0();  // the slot is read
-                issue_next(slot);
             }
             ++done;
             if (++slot == S) slot = 0;
         }
-        if (u > 0) lds_barrier();  // the last unit's sums are read
+        const int64_t m0 = unit_m0(u), n0 = unit_n0(u);
 #pragma unroll
-        for (int j = 0; j < NB; ++j)
+        for (int j0 = 0; j0 < NB; j0 += PJ) {
+            if (u + j0 > 0) lds_barrier();  // the last partial sums are read
 #pragma unroll
-            for (int i = 0; i < MB; ++i)
+            for (int j = 0; j < PJ; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    part[wave * kPart + (i * 16 + 4 * g + r) * BN + j * 16 + r16] = acc[j][i][r];
-        s_waitcnt_lgkm0();
-        lds_barrier();
+                for (int i = 0; i < MB; ++i)
 #pragma unroll
-        for (int e0 = 0; e0 < kPart; e0 += T) {
-            const int e = e0 + tid;
-            const int row = e / BN, col = u * BN + e % BN;
-            const int64_t n = (int64_t)(first + u * stride) * BN + e % BN;
-            if (e < kPart && row < a.rows && n < a.columns) {
-                const int64_t idx = row * a.columns + n;
-                if constexpr (WK == kW8A8) {
-                    unsigned sum = 0;
+                    for (int r = 0; r < 4; ++r)
+                        part[wave * kPart + (i * 16 + 4 * g + r) * PN + j * 16 + r16] = acc[j0 + j][i][r];
+            s_waitcnt_lgkm0();
+            lds_barrier();
 #pragma unroll
-                    for (int k = 0; k < KW; ++k) sum += (unsigned)part[k * kPart + e];
-                    if (a.acc_dump) a.acc_dump[idx] = (int)sum;
-                    float o;
-                    {
-                        // crates/omni-kernel/src/int8_matmul.rs:156-158: wrapping
-                        // int32, then two multiplies and the bias, each rounded.
+            for (int e0 = 0; e0 < kPart; e0 += T) {
+                const int e = e0 + tid;
+                const int row = e / PN, c = j0 * 16 + e % PN;
+                const int64_t m = m0 + row, n = n0 + c;
+                if (e < kPart && m < a.rows && n < a.columns) {
+                    const int64_t idx = m * a.columns + n;
+                    const int col = u * BN + c;
+                    if constexpr (WK == kW8A8) {
+                        unsigned sum = 0;
+#pragma unroll
+                        for (int k = 0; k < KW; ++k) sum += (unsigned)part[k * kPart + e];
+                        if (a.acc_dump) a.acc_dump[idx] = (int)sum;
+                        const int srow_i = (MT ? u * BM : 0) + row;
+                        float o;
+                        {
+                            // crates/omni-kernel/src/int8_matmul.rs:156-158: wrapping
+                            // int32, then two multiplies and the bias, each rounded.
 #pragma clang fp contract(off)
-                        const int centered = (int)(sum - (unsigned)s_sum[row] * (unsigned)s_zero[col]);
-                        const float t = (float)centered * s_scale[row];
-                        o = t * s_ws[col] + s_bias[col];
-                    }
-                    if (a.out_f16)
-                        static_cast<_Float16*>(a.out)[idx] = (_Float16)o;
-                    else
-                        static_cast<float*>(a.out)[idx] = o;
-                } else {
-                    float sum = 0.0f;
+                            const int centered = (int)(sum - (unsigned)s_sum[srow_i] * (unsigned)s_zero[col]);
+                            const float t = (float)centered * s_scale[srow_i];
+                            o = t * s_ws[col] + s_bias[col];
+                        }
+                        if (a.out_f16)
+                            static_cast<_Float16*>(a.out)[idx] = (_Float16)o;
+                        else
+                            static_cast<float*>(a.out)[idx] = o;
+                    } else {
+                        float sum = 0.0f;
 #pragma unroll
-                    for (int k = 0; k < KW; ++k) sum += part[k * kPart + e];
-                    static_cast<_Float16*>(a.out)[idx] = (_Float16)(sum * s_ws[col] + s_bias[col]);
+                        for (int k = 0; k < KW; ++k) sum += part[k * kPart + e];
+                        static_cast<_Float16*>(a.out)[idx] = (_Float16)(sum * s_ws[col] + s_bias[col]);
+                    }
                 }
             }
+            s_waitcnt_lgkm0();  // before the next barrier
         }
-        s_waitcnt_lgkm0();  // before the next unit's barrier
     }
 }
 
-template <int WK, int MB, int NB, int XC, int S, int KW, int TB>
+template <int WK, int MB, int NB, int XC, int S, int KW, int TB, bool MT = false>
 hipError_t launch_stream_cfg(const RowsArgs& a, int64_t cus, hipStream_t stream) {
-    const int64_t units = (a.columns + 16 * NB - 1) / (16 * NB);
-    constexpr int64_t kMost = kStreamColumns / (16 * NB);
+    const int64_t tiles_m = MT ? (a.rows + 16 * MB - 1) / (16 * MB) : 1;
+    const int64_t units = (a.columns + 16 * NB - 1) / (16 * NB) * tiles_m;
+    constexpr int64_t kMost = stream_units(NB, MT);
     const int64_t least = (units + kMost - 1) / kMost;
     // As many workgroups as are resident at once: two per CU where LDS allows.
-    constexpr int kLds = KW * (S * (16 * NB * TB / 1024 + XC) + MB * NB) * 1024 + 12 * kStreamColumns + 128 * MB;
+    constexpr int kLds = KW * (S * (16 * NB * TB / 1024 + XC) + MB * NB) * 1024 + 12 * 16 * NB * (int)kMost + 128 * MB;
     const int64_t cap = cus * (KW == 4 && kLds <= 80 * 1024 ? 2 : 1);
     const int64_t grid = units < cap ? units : (least > cap ? least : cap);
-    if (grid > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((rows_stream_kernel<WK, MB, NB, XC, S, KW, TB>), dim3((unsigned)grid), dim3(64 * KW), 0, stream, a);
+    if (grid > 0x7fffffff || units > 0x7fffffff) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((rows_stream_kernel<WK, MB, NB, XC, S, KW, TB, MT>), dim3((unsigned)grid), dim3(64 * KW), 0,
+                       stream, a);
     return hipGetLastError();
 }
-
-}  // namespace
-
-namespace {
 
 // Blocks of 16 columns outnumber the CUs.
 bool is_wide(int64_t columns, int64_t cus) { return columns > 16 * cus; }
@@ -391,6 +445,27 @@ hipError_t launch_even(const RowsArgs& a, hipStream_t st) {
                 : launch_stream_cfg<WK, 4, 1, 8, 2, 4, 128>(a, cus, st);
 }
 
+// Row blocks per workgroup above 64 rows: the rows spread evenly over the
+// fewest tiles of at most 64 (then 3 or 4 blocks of 16).
+int row_blocks(int64_t rows) {
+    const int64_t tiles = (rows + 63) / 64;
+    return (int)(((rows + tiles - 1) / tiles + 15) / 16);
+}
+int64_t row_units(int64_t rows, int64_t columns, int nb) {
+    const int64_t bm = 16 * row_blocks(rows);
+    return (rows + bm - 1) / bm * ((columns + 16 * nb - 1) / (16 * nb));
+}
+
+// More than 64 rows: tiles of 48 or 64 rows by 16 NB columns, K split over
+// four waves that each own a ring.
+template <int WK, int NB, int TB>
+hipError_t launch_tiles(const RowsArgs& a, hipStream_t st) {
+    const int64_t cus = num_cus();
+    constexpr int kXC = 16 * TB * x_bytes(WK) / 1024;  // copies per 16 rows
+    return row_blocks(a.rows) == 3 ? launch_stream_cfg<WK, 3, NB, 3 * kXC, 2, 4, TB, true>(a, cus, st)
+                                   : launch_stream_cfg<WK, 4, NB, 4 * kXC, 2, 4, TB, true>(a, cus, st);
+}
+
 RowsArgs f16_args(const W8A16Args& w, int64_t row_bytes) {
     RowsArgs a{};
     a.x = reinterpret_cast<const uint8_t*>(w.x);
@@ -411,10 +486,10 @@ constexpr int64_t kMaxRowBytes = 1 << 18;
 }  // namespace
 
 bool w8a8_rows_fits(const W8A8Args& a) {
-    return a.rows <= 64 && a.width % 16 == 0 && a.width >= 16 && a.width <= kMaxRowBytes;
+    return a.rows <= 4096 && a.width % 16 == 0 && a.width >= 16 && a.width <= kMaxRowBytes;
 }
 
-hipError_t launch_w8a8_rows(const W8A8Args& w, hipStream_t st) {
+hipError_t launch_w8a8_rows(const W8A8Args& w, int nb, hipStream_t st) {
     if (w.rows == 0 || w.columns == 0) return hipSuccess;
     RowsArgs a{};
     a.x = w.x;
@@ -430,7 +505,24 @@ hipError_t launch_w8a8_rows(const W8A8Args& w, hipStream_t st) {
     a.bias = w.bias;
     a.acc_dump = w.acc_dump;
     a.out_f16 = w.out_f16;
-    return launch_even<kW8A8>(a, st);
+    if (a.rows <= 64) return launch_even<kW8A8>(a, st);
+    return nb == 2 ? launch_tiles<kW8A8, 2, 128>(a, st) : launch_tiles<kW8A8, 4, 128>(a, st);
+}
+
+// Time in us of 65 rows and more in blocks of 32 or 64 columns, fitted to 65
+// to 1024 rows of thirteen K x N (1152 ... 14336 x 1152 ... 28672): each round
+// of one tile per CU costs a fixed part and its K loop (within 10 % of 64 of
+// the 78 timings, 20 % of the rest).
+double w8a8_rows_us(int64_t rows, int64_t columns, int64_t width, int* nb) {
+    const int64_t cus = num_cus();
+    const int mb = row_blocks(rows);
+    auto us = [&](int n, double fixed, double per_k) {
+        const int64_t rounds = (row_units(rows, columns, n) + cus - 1) / cus;
+        return 5.0 + (double)rounds * (fixed + per_k * (double)width * (mb + n) / (4 + n));
+    };
+    const double t2 = us(2, 1.3, 0.0015), t4 = us(4, 2.1, 0.00206);
+    *nb = t2 < t4 ? 2 : 4;
+    return t2 < t4 ? t2 : t4;
 }
 
 // Five to 64 rows, against the skinny kernels and the GEMM (w8a16.hip):
@@ -471,6 +563,11 @@ hipError_t launch_w8a16_rows(const W8A16Args& w, hipStream_t st) {
     const RowsArgs a = f16_args(w, w.width);
     const int64_t cus = num_cus();
     const bool wide = is_wide(a.columns, cus);
+    // Blocks of 32 columns while one round holds them (128 rows of 4096 x 4096
+    // 14.9 against 19.0 us), else of 64.
+    if (w.rows > 64)
+        return row_units(a.rows, a.columns, 2) <= cus ? launch_tiles<kW8A16, 2, 64>(a, st)
+                                                      : launch_tiles<kW8A16, 4, 64>(a, st);
     // Wide: two four-wave workgroups per CU, or from K = 4096 and 9 rows on
     // blocks of 32 columns (8 rows of 4096 x 6144 7.7 against 8.8 us, of 1536
     // x 17920 9.7 against 8.7; 16 rows of 4096 x 14336 16.5 against 21.4).

@@ -1507,7 +1507,7 @@ int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width) {
     a.columns = columns;
     a.width = width;
     if (!ring_offsets_fit(a)) return 0;
-    if (w8a8_tile_override() == 0 && w8a8_rows_fits(a)) return 0;  // no split there
+    if (w8a8_tile_override() == 0 && rows <= 64 && w8a8_rows_fits(a)) return 0;  // no split there
     const int sp = w8a8_auto_splits(rows, columns, width, num_cus());
     return sp > 1 ? (int64_t)sp * rows * columns : 0;
 }
@@ -1527,17 +1527,16 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream) {
         case 16: return launch_pair<192>(a, stream);
         case 17: return launch_pair<128>(a, stream, w8a8_split_override());
         case 19: return launch_ring8_256(a, stream);
-        case 30:
-            if (w8a8_rows_fits(a)) return launch_w8a8_rows(a, stream);
-            break;
-        case 0:
-            // Up to 64 rows the weights' stream is all that counts: on every
-            // shape measured (rows.hip) the streaming kernel is ahead of the
-            // 256-row tiles below.
-            if (w8a8_rows_fits(a)) return launch_w8a8_rows(a, stream);
+        case 30:  // the streaming kernels in blocks of 32 columns, 31: of 64
+        case 31:
+            if (w8a8_rows_fits(a)) return launch_w8a8_rows(a, w8a8_tile_override() == 30 ? 2 : 4, stream);
             break;
         default: break;
     }
+    const bool pinned = w8a8_tile_override() != 0;
+    // Up to 64 rows the weights' stream is all that counts: on every shape
+    // measured (rows.hip) the streaming kernel is ahead of 256-row tiles.
+    if (!pinned && a.rows <= 64 && w8a8_rows_fits(a)) return launch_w8a8_rows(a, 0, stream);
     // Cost model, fitted to MI355X timings of every candidate on ten shapes
     // (the BASELINE GEMM shapes and the reference's 256-row benchmark shapes;
     // codes of N(0,1) rows and uniform weights rotated past the MALL, f32
@@ -1560,8 +1559,22 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream) {
         return (double)(bm * bn) * (c * K + e) * rounds;
     };
     struct Cand { double t; int id; };
+    // More rows on small matrices: the streaming kernels' tiles, where their
+    // time by w8a8_rows_us is below 0.95 of the choice below. That choice's
+    // time, fitted to 78 timings (65 to 1024 rows, thirteen K x N of 1152 ...
+    // 14336 x 1152 ... 28672) where its tiles leave CUs idle: the cost model's
+    // (in fs) plus 2.5 us unsplit, 1.2 times it for the register-staged
+    // kernels, and for split K and its reduction a line in the weights' MB
+    // and the rows. On 117 timings (those shapes at 65 to 1024 rows) the rule's
+    // choice is within 6 % of the fastest on 107 and 18 % off at worst; the
+    // tiles are up to 5 times faster (65 rows of 4304 x 1152).
+    int tiles_nb = 0;
+    const double tiles_us =
+        !pinned && w8a8_rows_fits(a) ? w8a8_rows_us(a.rows, a.columns, a.width, &tiles_nb) / 0.95 : 1e30;
     if (a.width % 64 != 0 || !ring_offsets_fit(a)) {
         // Register-staged kernels: any K % 16 == 0.
+        const double c128 = cost(308.0, 250000.0, 256, 128), c192 = cost(280.5, 227212.0, 256, 192);
+        if (tiles_us < 1.2e-9 * (c128 < c192 ? c128 : c192)) return launch_w8a8_rows(a, tiles_nb, stream);
         return cost(308.0, 250000.0, 256, 128) < cost(280.5, 227212.0, 256, 192) ? launch_bn<128, 2>(a, stream)
                                                                                  : launch_bn<192, 2>(a, stream);
     }
@@ -1569,7 +1582,12 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream) {
     const int sp = w8a8_auto_splits(a.rows, a.columns, a.width, cus);
     if (sp > 1) {
         const int64_t tiles = ((a.rows + 255) / 256) * ((a.columns + 127) / 128);
-        if (fit_splits(a, tiles, (int)kt, sp) > 1) return launch_pair<128>(a, stream, sp);
+        if (fit_splits(a, tiles, (int)kt, sp) > 1) {
+            // The GEMM and its reduction, us.
+            const double m = (double)a.rows / 256.0, mb = 1e-6 * K * (double)a.columns;
+            if (tiles_us < 12.0 + 0.22 * mb + m * (5.0 + 0.09 * mb)) return launch_w8a8_rows(a, tiles_nb, stream);
+            return launch_pair<128>(a, stream, sp);
+        }
     }
     Cand best{cost(243.7, 117070.0, 256, 192), 16};
     auto consider = [&](bool ok, double t, int id) {
@@ -1584,6 +1602,7 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream) {
     // shapes on the 256 x 192 pair ring, which stays faster there.
     consider(s4, cost(240.7, 163216.0, 256, 256), 19);
     consider(!s4 && s3, cost(250.7, 210425.0, 256, 256), 14);
+    if (tiles_us < 1e-9 * best.t + 2.5) return launch_w8a8_rows(a, tiles_nb, stream);
     switch (best.id) {
         case 19: return launch_ring8_256(a, stream);
         case 14: return launch_ring<256, 3>(a, stream);

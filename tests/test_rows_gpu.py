@@ -30,6 +30,28 @@ def host(t):
     (3, 512, 4097), (7, 1152, 4112), (16, 400, 5001), (31, 528, 4100), (47, 384, 4129), (64, 656, 4128),
     (2, 64, 140001), (13, 32, 140001), (64, 48, 131104)])
 def test_w8a8_stream_bit_exact(oracle, rows, width, columns):
+    w8a8_case(oracle, rows, width, columns)
+
+
+# More than 64 rows in tiles of 48 and 64 by 32 (30) and 64 (31) columns: ragged
+# in each direction, partial K tiles, more units than one workgroup per CU
+# holds, more than eight units per workgroup.
+@pytest.mark.parametrize("tile", ["30", "31"])
+@pytest.mark.parametrize("rows,width,columns", [
+    (65, 64, 33), (96, 144, 64), (97, 1040, 65), (128, 528, 130), (129, 16, 31), (190, 2048, 100), (256, 272, 515),
+    (300, 96, 6000), (1000, 208, 1100), (2049, 48, 8300)])
+def test_w8a8_tiles_bit_exact(oracle, rows, width, columns, tile, knobs):
+    knobs.set("OMNI_W8A8_TILE", tile)
+    w8a8_case(oracle, rows, width, columns)
+
+
+# The default route of small matrices.
+@pytest.mark.parametrize("rows,width,columns", [(65, 4304, 1152), (100, 1536, 1536), (200, 1152, 777)])
+def test_w8a8_tiles_by_default(oracle, rows, width, columns):
+    w8a8_case(oracle, rows, width, columns)
+
+
+def w8a8_case(oracle, rows, width, columns):
     rng = np.random.default_rng(rows * 7 + width + columns)
     codes = rng.integers(-128, 128, (rows, width), dtype=np.int8)
     w = rng.integers(-128, 128, (columns, width), dtype=np.int8)
@@ -64,7 +86,8 @@ def close(got, want):
     (1, 18944, 40), (4, 16400, 33), (3, 4112, 17), (4, 1552, 8195), (5, 16, 7), (6, 1040, 100), (8, 4624, 4100),
     (8, 1168, 4112), (9, 4112, 64), (16, 240, 31), (13, 4096, 4113), (16, 528, 9000), (17, 64, 16), (32, 1104, 50),
     (31, 336, 4130), (33, 272, 40), (48, 1040, 300), (47, 368, 4100), (49, 144, 30), (64, 2064, 70), (63, 400, 4101),
-    (24, 32, 131200)])
+    (24, 32, 131200), (65, 1536, 33), (96, 80, 64), (97, 4608, 65), (128, 208, 130), (192, 4304, 100), (256, 64, 515),
+    (300, 48, 2100), (130, 1168, 4300), (2049, 16, 900)])
 def test_w8a16_stream(rows, width, columns):
     rng = np.random.default_rng(rows + 3 * width + columns)
     x = rng.standard_normal((rows, width)).astype(np.float16)
