@@ -77,6 +77,9 @@ def quantize_rows(x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Te
 
     x: [rows, width] f32 or f16 on the GPU -> (codes int8 [rows, width],
     row_scale f32 [rows], row_sum int32 [rows])."""
+    direct = (_lib._host or _lib.host()).quantize_rows(x)
+    if direct is not NotImplemented:
+        return direct
     if x.dim() != 2:
         raise ValueError("x must be 2-D")
     device = _require_gpu(x)
@@ -119,6 +122,11 @@ def w8a8_gemm(codes: torch.Tensor, row_scale: torch.Tensor, row_sum: Optional[to
     (may be None when w_zero is None); w_scale f32 [columns]; w_zero int32
     [columns]; bias f32 [columns]. Returns out (and the int32 accumulators if
     acc_dump)."""
+    if not acc_dump and lowering == OMNI_LOWERING_AUTO and out_dtype in (torch.float32, torch.float16):
+        direct = (_lib._host or _lib.host()).w8a8_gemm(codes, row_scale, row_sum, w, w_scale, w_zero, bias,
+                                                       out_dtype is torch.float16)
+        if direct is not NotImplemented:
+            return direct
     device = _require_gpu(codes, row_scale, row_sum, w, w_scale, w_zero, bias)
     if codes.dim() != 2 or codes.dtype != torch.int8:
         raise ValueError("codes must be int8 [rows, width]")
@@ -169,6 +177,9 @@ def try_int8_gemm(x: torch.Tensor, w_packed: torch.Tensor, w_scale: torch.Tensor
     (:525-526; f16 is passed through, since it is exact in f32); integer
     inputs may be int32 or int64 (int64 is truncated to int32 as read_i32,
     :587-595, does)."""
+    direct = (_lib._host or _lib.host()).try_int8_gemm(x, w_packed, w_scale, w_zero)
+    if direct is not NotImplemented:
+        return direct
     rows, width = x.shape
     columns = w_scale.shape[0]
     if width % 4 != 0 or w_packed.shape[0] != columns * width // 4 or w_zero.shape[0] != columns:
@@ -202,6 +213,9 @@ def w8a16_linear(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor,
     x f16 [rows, width] (leading dims are flattened), w int8 [columns, width],
     scale/bias f16 [columns] -> f16 [..., columns]. Decode shapes (rows <= 4)
     run the HBM-bound GEMV, larger ones the fp16-MFMA GEMM."""
+    direct = (_lib._host or _lib.host()).w8a16_linear(x, w, scale, bias)
+    if direct is not NotImplemented:
+        return direct
     lead = x.shape[:-1]
     width = x.shape[-1]
     x2 = x.reshape(-1, width)
@@ -239,6 +253,9 @@ def w4a16_linear(x: torch.Tensor, w_packed: torch.Tensor, scale: torch.Tensor,
     x f16 [..., width]; w_packed uint8 [columns, width // 2] (two values per
     byte, low nibble first, stored plus 8); scale bf16 [columns, width // group];
     bias f16 [columns] -> f16 [..., columns]."""
+    direct = (_lib._host or _lib.host()).w4a16_linear(x, w_packed, scale, bias, group)
+    if direct is not NotImplemented:
+        return direct
     lead = x.shape[:-1]
     width = x.shape[-1]
     x2 = x.reshape(-1, width)

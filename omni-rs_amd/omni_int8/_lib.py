@@ -61,6 +61,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_host = None
 
 
 class OmniError(RuntimeError):
@@ -95,3 +96,20 @@ def check(status: int) -> int:
     if status not in (OMNI_OK, OMNI_NOT_HANDLED):
         raise OmniError(status, last_error())
     return status
+
+
+def host():
+    """The package's direct calls (csrc/host.cpp, built beside the library),
+    bound to the same library as lib(). Each returns NotImplemented where its
+    Python wrapper has to do the work."""
+    global _host
+    if _host is None:
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise OmniError(OMNI_BAD_ARGUMENT,
+                            f"omni_int8/_host.so does not load ({e}); build it with `make -C omni-rs_amd`") from None
+        handle = lib()
+        module.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in SIGNATURES})
+        _host = module
+    return _host

@@ -232,6 +232,10 @@ class Int8Linear:
         if dims[-1] != self.input:
             # convrot.rs:84 asserts the width
             raise ValueError(f"ConvRot input width {dims[-1]} != {self.input}")
+        direct = (_lib._host or _lib.host()).convrot_linear(x, self.packed, self.scale, self.zero,
+                                                            self.precision is torch.float16)
+        if direct is not NotImplemented:
+            return direct
         rows = int(np.prod(dims[:-1])) if len(dims) > 1 else 1
         flat = x.reshape(rows, self.input)
         if flat.dtype not in (torch.float16, torch.float32):
@@ -242,7 +246,8 @@ class Int8Linear:
             if t.device != device:
                 raise _lib.OmniError(_lib.OMNI_BAD_ARGUMENT, "tensors live on different devices")
         L = _lib.lib()
-        ws_bytes = L.omni_try_int8_gemm_workspace_size(rows, self.input)
+        # With room for the split-K partial sums the GEMM splits K where that pays.
+        ws_bytes = L.omni_try_int8_gemm_split_workspace_size(rows, self.scale.numel(), self.input)
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
         out = torch.empty((rows, self.output), dtype=self.precision, device=device)
         st = _lib.check(L.omni_convrot_linear(

@@ -31,6 +31,9 @@ __all__ = ["depth_try_linear", "tensorops_try_linear"]
 
 
 def _run(entry: str, x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    direct = (_lib._host or _lib.host()).f16_linear(entry == "omni_f16_gemm", x, w)
+    if direct is not NotImplemented:
+        return direct
     if x.device.type != "cuda" or w.device != x.device:
         return None
     if x.dim() < 1 or w.dim() != 2 or x.dtype != torch.float16 or w.dtype != torch.float16:
