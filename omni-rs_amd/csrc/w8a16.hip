@@ -2391,23 +2391,24 @@ hipError_t launch_f16_mfma(const W8A16Args& a, hipStream_t stream) {
         default: break;
     }
     const int64_t cus = cu_count();
-    // Eight-wave rings (two waves per SIMD, each 64 x 128 or 64 x 64) on
-    // 64-element K tiles (whole 128-byte lines of x and W): 256 x 256 tiles
-    // in a 2-stage ring or 256 x 128 tiles in a 3-stage ring, whichever a
-    // rounds cost model picks: tiles run in rounds of one per CU, a partial
-    // last round with fill f costs 0.7 + 0.3 f of a full one, and a 256 x 256
-    // tile costs 1.80 times a 256 x 128 one (MI355X, best of three:
-    // 4096 x 4096 x 12288 334.5 / 365.0 us, torch.matmul 321.0; 4352 x 4096 x
-    // 12288 408.1 / 422.8, torch.matmul 418.7; 2048 x 4096 x 4096 80.4 /
-    // 64.6, torch.matmul 62.5; the 256 x 256 ring on 32-element K tiles
-    // 356.9 / 433.7 / 79.4).
+    // Rings on 64-element K tiles (whole 128-byte lines of x and W): eight
+    // waves on 256 x 256 tiles in two stages or on 256 x 128 in three, four
+    // waves on 128 x 128 in three, whichever a rounds cost model picks: tiles
+    // run in rounds of one per CU, a partial last round with fill f costs
+    // 0.7 + 0.3 f of a full one, and a tile 1.80 and 0.56 times a 256 x 128 one
+    // (MI355X: a full round at K = 4096 takes 122, 67.6 and 37.8 us; 4096 x
+    // 4096 x 12288 365 / 405 / 453 us, torch.matmul 320; 2048 x 4096 x 4096 88
+    // / 67 / 74, torch.matmul 64; 512 x 6592 x 6080 133 / 93 / 62,
+    // torch.matmul 60; 300 x 4096 x 4096 73 / 45 / 29, torch.matmul 23).
     if (ring_ok && a.width >= 3072) {
-        auto rounds = [&](int64_t bn) {
-            const int64_t tiles = ((a.rows + 255) / 256) * ((a.columns + bn - 1) / bn);
+        auto rounds = [&](int64_t bm, int64_t bn) {
+            const int64_t tiles = ((a.rows + bm - 1) / bm) * ((a.columns + bn - 1) / bn);
             const int64_t full = tiles / cus, rem = tiles % cus;
             return (double)full + (rem ? 0.7 + 0.3 * (double)rem / (double)cus : 0.0);
         };
-        if (1.80 * rounds(256) <= rounds(128)) return launch_ring16_cfg<256, 256, 16, 4, 2, 2, 1, 8>(a, stream);
+        const double t256 = 1.80 * rounds(256, 256), t128 = rounds(256, 128), t64 = 0.56 * rounds(128, 128);
+        if (t64 < t128 && t64 < t256) return launch_ring16_cfg<128, 128, 16>(a, stream);
+        if (t256 <= t128) return launch_ring16_cfg<256, 256, 16, 4, 2, 2, 1, 8>(a, stream);
         return launch_ring16_cfg<256, 128, 16, 4, 3, 2, 1, 8>(a, stream);
     }
     const int64_t big_tiles = ((a.rows + 127) / 128) * ((a.columns + 127) / 128);
