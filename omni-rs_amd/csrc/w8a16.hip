@@ -2009,6 +2009,54 @@ hipError_t launch_w8a16_skinny(const W8A16Args& a, hipStream_t stream) { return 
 // the call brings a workspace. Both are tuning knobs (omni::knob).
 int w8a16_tile_override() { return knob(Knob::W8A16Tile, 0); }
 
+// One ring kernel's time in us, fitted to measurements: units (tiles, times
+// the splits of K) run in rounds of occ per CU, a full round takes a + b K /
+// splits / 1000, a partial last one with fill f p + (1 - p) f of that, a launch
+// t0, and a split's reduction r0 + r1 us per million of its partial sums.
+// unsplit and split weigh the estimate where its error has a sign. r0 = 0: not
+// split.
+struct RingFit {
+    int id;  // as OMNI_W8A16_TILE and OMNI_W4A16_TILE number the rings
+    int bm, bn, occ;
+    double a, b, p, t0, r0, r1, unsplit, split;
+};
+struct RingChoice {
+    int id, splits;
+};
+
+// The ring and the split of K (up to 4 ways, or `override` ways) with the
+// least estimated time; ws_limited: only splits whose partial sums a.partial
+// holds.
+RingChoice pick_ring(const RingFit* fits, size_t count, const W8A16Args& a, int cus, bool ws_limited, int override) {
+    const int ktiles = (int)(a.width / 64);
+    RingChoice best{fits[0].id, 1}, forced{0, 0};
+    double best_t = 0.0, forced_t = 0.0;
+    for (size_t i = 0; i < count; ++i) {
+        const RingFit& f = fits[i];
+        const int64_t tiles = ((a.rows + f.bm - 1) / f.bm) * ((a.columns + f.bn - 1) / f.bn);
+        auto time = [&](int sp) {
+            const int64_t units = tiles * sp, slots = (int64_t)cus * f.occ;
+            const int64_t full = units / slots, rem = units % slots;
+            const double rounds = (double)full + (rem ? f.p + (1.0 - f.p) * (double)rem / (double)slots : 0.0);
+            double t = f.t0 + rounds * (f.a + 1e-3 * f.b * (double)a.width / sp);
+            if (sp == 1) return t * f.unsplit;
+            return (t + f.r0 + 1e-6 * f.r1 * sp * (double)a.rows * (double)a.columns) * f.split;
+        };
+        auto splits = [&](int sp) {  // every split non-empty, and room for its sums
+            if (sp > ktiles || (sp - 1) * ((ktiles + sp - 1) / sp) >= ktiles) return false;
+            return !ws_limited || fit_splits(a, ktiles, sp) == sp;
+        };
+        for (int sp = 1; sp <= (f.r0 > 0.0 ? 4 : 1); ++sp) {
+            if (sp > 1 && !splits(sp)) continue;
+            const double t = time(sp);
+            if (best_t == 0.0 || t < best_t) best_t = t, best = {f.id, sp};
+        }
+        if (override > 1 && f.r0 > 0.0 && (forced_t == 0.0 || time(override) < forced_t))
+            forced_t = time(override), forced = {f.id, override};
+    }
+    return override > 1 && (!ws_limited || fit_splits(a, ktiles, override) > 1) ? forced : best;
+}
+
 // The kernel and split count launch_w8a16_mfma runs for a shape: cfg as
 // OMNI_W8A16_TILE numbers them (0: the register-staged kernels), splits > 1
 // for split K (needs splits * rows * columns floats of partial sums).
@@ -2029,85 +2077,27 @@ W16Plan plan_w8a16(const W8A16Args& a, int cus, bool ws_limited) {
         const int64_t big_tiles = ((a.rows + 127) / 128) * ((a.columns + 127) / 128);
         return {big_tiles >= 512 ? 1 : 2, 1};
     }
-    auto with_splits = [&](int cfg) { return W16Plan{cfg, split_override > 1 ? split_override : 1}; };
-    // Split K (f32 partial sums, one reduction launch) when even 64 x 128
-    // tiles leave CUs idle and K is long: 128 x 128 tiles two per CU, K split
-    // 2..4 ways to about one unit per CU (MI355X, weights rotated past the
-    // MALL: 1024 x 8960 -> 1536 46.9 us against 54.2 unsplit, 256 x 12288 ->
-    // 4096 41.0 against 76.7, 256 x 4096 -> 4096 24.6 against 28.5). On K =
-    // 1536 the partial sums' traffic costs more than the split saves.
-    const int64_t tiles64 = ((a.rows + 63) / 64) * ((a.columns + 127) / 128);
-    if (a.width >= 4096 && tiles64 < cus) {
-        // K >= 8192 with as many 128 x 192 tiles as divide the CUs 2-4 ways:
-        // those tiles split that many ways fill every CU exactly once
-        // (config 5's down projection, 1024 x 8960 -> 1536: 64 tiles, four
-        // splits, 40.9 us against 45.9 on 128 x 128 tiles split two ways; on
-        // K = 4096, or splits that leave CUs idle, the rule below wins).
-        const int64_t tiles192 = ((a.rows + 127) / 128) * ((a.columns + 191) / 192);
-        if (a.width >= 8192 && split_override <= 1 && cus % tiles192 == 0) {
-            const int sp = (int)(cus / tiles192);
-            if (sp >= 2 && sp <= 4 && (!ws_limited || fit_splits(a, (int)(a.width / 64), sp) == sp))
-                return {21, sp};
-        }
-        const int64_t tiles128 = ((a.rows + 127) / 128) * ((a.columns + 127) / 128);
-        const int64_t want = cus / tiles128;
-        const int sp = split_override > 1 ? split_override : (int)(want < 2 ? 2 : want > 4 ? 4 : want);
-        if (!ws_limited || fit_splits(a, (int)(a.width / 64), sp) > 1) return {10, sp};
-    }
-    // Cost model over the one-workgroup-per-CU rings, fitted to MI355X
-    // timings (weights rotated past the MALL) of every ring on twelve prefill
-    // shapes, M 512..4096, K 1536..4096, N 1536..17920: tiles run in rounds
-    // of one per CU, a round costs BM * BN * (c * K + e), a partial last
-    // round with fill f costs 0.7 + 0.3 f of a full one. It picks within
-    // 1.2 % of the fastest ring on all twelve (the fixed rules it replaces:
-    // up to 40 % off). Candidates: 256 x 192 (four waves), 128 x 256 and
-    // 256 x 256 with eight waves (two per SIMD; the 256 x 256 one measured
-    // 4-15 % faster than the four-wave 256 x 256 ring with the waves side by
-    // side along N on seven shapes, so it takes that ring's fit less 4 %).
-    struct Cand {
-        double t;
-        int id;
-        int64_t tiles;
+    // MI355X fits over 150 shapes (65 to 4352 rows, K 1024 ... 14336, N 1024 ...
+    // 18944, every ring and split; median error 2-6 %). The choice by them is
+    // within 2 % of the fastest on average, where the rules it replaces (one
+    // model for the one-per-CU rings, hand-set lines for splits and small
+    // tiles) were 9 % off: 582 x 7680 -> 3264 41 us against 69 (128 x 192 tiles
+    // split three ways), 109 x 3968 -> 2112 14 against 22; config 5's gate/up
+    // (128 x 320 tiles) and down (128 x 192 split four ways) are as before.
+    static constexpr RingFit kFits[] = {
+        {5, 128, 128, 1, 4.67, 7.53, 0.69, 1.97, 0.0, 0.00, 0.98, 1.00},
+        {8, 64, 128, 1, 2.63, 5.39, 0.83, 2.13, 0.0, 0.00, 1.10, 1.00},
+        {9, 256, 192, 1, 10.32, 17.21, 0.73, 4.28, 1.3, 0.81, 1.00, 0.96},
+        {10, 128, 128, 2, 5.25, 14.94, 0.30, 3.45, 2.8, 0.87, 1.02, 1.04},
+        {12, 64, 128, 3, 4.47, 14.73, 0.24, 2.81, 2.8, 0.78, 0.98, 1.00},
+        {16, 128, 256, 1, 5.66, 13.01, 0.65, 2.56, 2.7, 0.82, 1.00, 1.00},
+        {18, 256, 256, 1, 15.52, 20.34, 0.67, 0.00, 1.8, 0.81, 1.00, 1.06},
+        {19, 128, 320, 1, 10.28, 15.39, 0.73, 1.80, 2.3, 0.75, 1.00, 1.00},
+        {20, 64, 192, 1, 3.95, 7.29, 0.83, 2.11, 0.0, 0.00, 1.00, 1.00},
+        {21, 128, 192, 1, 5.34, 9.82, 0.67, 3.71, 2.4, 0.89, 1.00, 1.06},
     };
-    auto cost = [&](int id, double c, double e, int64_t bm, int64_t bn) {
-        const int64_t tiles = ((a.rows + bm - 1) / bm) * ((a.columns + bn - 1) / bn);
-        const int64_t full = tiles / cus, rem = tiles % cus;
-        const double rounds = (double)full + (rem ? 0.7 + 0.3 * (double)rem / (double)cus : 0.0);
-        return Cand{(double)(bm * bn) * (c * (double)a.width + e) * rounds, id, tiles};
-    };
-    // (The 256 x 256 and 256 x 192 fits are scaled by 0.94 and 0.90: spreading
-    // the code conversion over the MFMA slots made those rings 3-14 % and
-    // 6-16 % faster on eight of these shapes, the 128 x 256 one 0-3 % slower.
-    // The 256 x 256 candidate is then the eight-wave ring with two waves
-    // along M (each 128 x 64, half the conversions per MFMA of the 64 x 128
-    // one): 0.93-0.96 of that one's time on five shapes, so 0.95 of its fit.)
-    // 128 x 320 (four waves of 64 x 160; 2 BM + BN = 9 x 64 stage rows, so
-    // the copies divide over the waves) gives the M = 1024 and 2048 shapes
-    // 8 x 28 / 16 x 28 tiles where 256 x 192 leaves a quarter of the CUs idle
-    // (1024 x 1536 -> 8960: 188 tiles): fitted on MI355X at K = 1536 and
-    // 4096 (1024 x K -> 8960: 36.8 / 79.1 us), it changes the pick on eight
-    // of 38 swept shapes, each 5-13 % faster (1024 x 1536 -> 17920: 72.5
-    // against 83.8 us), and on no other.
-    Cand best = cost(18, 0.3184, 358.8, 256, 256);
-    for (const Cand& c : {cost(9, 0.3846, 359.2, 256, 192), cost(16, 0.4289, 201.6, 128, 256),
-                          cost(19, 0.4186, 291.4, 128, 320)})
-        if (c.t < best.t) best = c;
-    // At most half a round of tiles and K >= 8192: split that ring's tiles
-    // 2-4 ways to about one unit per CU (1024 x 18944 -> 3584: 128 x 256
-    // tiles split two ways 155.9-158.7 us, against 194.6 on 64 x 128 tiles
-    // three per CU; 1024 x 14336 -> 4096: 126.8 against 153.7 unsplit).
-    if (a.width >= 8192 && 2 * best.tiles <= cus) {
-        const int64_t want = cus / best.tiles;
-        const int sp = split_override > 1 ? split_override : (int)(want < 2 ? 2 : want > 4 ? 4 : want);
-        if (!ws_limited || fit_splits(a, (int)(a.width / 64), sp) > 1) return {best.id, sp};
-    }
-    if (2 * best.tiles >= cus) return with_splits(best.id);
-    // Fewer tiles than half the CUs: 64 x 128 tiles three workgroups per CU
-    // when they fit one round of those slots (config 5's 1024 x 1536 ->
-    // 1536 / 2048 / 512: 13.4 / 13.4 / 11.9 us against 20.9 / 20.8 / 19.9
-    // for 128 x 256), else 128 x 256.
-    if (tiles64 <= 3 * (int64_t)cus) return with_splits(12);
-    return with_splits(16);
+    const RingChoice c = pick_ring(kFits, sizeof(kFits) / sizeof(kFits[0]), a, cus, ws_limited, split_override);
+    return {c.id, c.splits};
 }
 
 int64_t w8a16_skinny_partial_elems(int64_t rows, int64_t columns, int64_t width) {
@@ -2286,42 +2276,21 @@ W4Plan plan_w4a16(const W8A16Args& a, int cus, bool ws_limited) {
         const int64_t big_tiles = ((a.rows + 127) / 128) * ((a.columns + 127) / 128);
         return {big_tiles >= 512 ? 1 : 2, 1};
     }
-    // Rings 256 x 256 (eight waves, each 128 x 64) / 256 x 128 / 128 x 128,
-    // each unsplit or with K split 2-4 ways, whichever a rounds cost model
-    // picks: units (tiles, or tiles x splits) run in rounds of one per CU, a
-    // partial last round with fill f costs 0.7 + 0.3 f of a full one, a full
-    // round costs c K' + e us for K' = K / splits (MI355X fits over M =
-    // 256..4096, K = 3584..18944: 0.02488 K' + 31.4, 0.01435 K' + 24.2,
-    // 0.0107 K' + 8.1), and a split adds its reduction, 1 us + (4 splits + 2)
-    // bytes per output at 3.5 TB/s; K < 4096 is not split. On seven long-K
-    // shapes its choice is within 5 % of the fastest of the ring/split
-    // choices measured on five and 13-14 % off on two (1024 x 8192 -> 4096,
-    // 1024 x 8960 -> 1536); against unsplit: 1024 x 14336 -> 4096 142 us
-    // against 182, 1024 x 8960 -> 1536 56 against 86.
-    const int ktiles = (int)(a.width / 64);
-    double best_t = 0.0;
-    W4Plan best{5, 1};
-    auto consider = [&](int id, int64_t bm, int64_t bn, double c, double e) {
-        const int64_t tiles = ((a.rows + bm - 1) / bm) * ((a.columns + bn - 1) / bn);
-        for (int sp = 1; sp <= 4; ++sp) {
-            if (sp > 1 && (a.width < 4096 || (ws_limited && fit_splits(a, ktiles, sp) != sp))) break;
-            const int64_t units = tiles * sp;
-            const int64_t full = units / cus, rem = units % cus;
-            const double rounds = (double)full + (rem ? 0.7 + 0.3 * (double)rem / (double)cus : 0.0);
-            double t = rounds * (c * (double)a.width / sp + e);
-            if (sp > 1) t += 1.0 + (4.0 * sp + 2.0) * (double)a.rows * (double)a.columns / 3.5e6;
-            if (best_t == 0.0 || t < best_t) {
-                best_t = t;
-                best = {id, sp};
-            }
-        }
+    // MI355X fits over 130 shapes (33 to 4352 rows, K 1024 ... 14336, N 1024 ...
+    // 18944, every ring and split; median error 3-6 %). The choice by them is
+    // within 1 % of the fastest on average and 4 % slower than before at worst,
+    // where the three rings it knew, split only from K = 4096 on, were 11 % off:
+    // 67 x 3328 -> 1664 16 us against 35, 191 x 2816 -> 1280 16 against 30 (128
+    // x 128 tiles two per CU, split four ways).
+    static constexpr RingFit kFits[] = {
+        {4, 256, 128, 1, 4.01, 15.18, 0.72, 7.28, 0.7, 1.24, 1.04, 0.98},
+        {5, 128, 128, 1, 1.65, 10.44, 0.77, 5.00, 2.2, 1.32, 1.02, 1.00},
+        {10, 128, 128, 2, 1.50, 19.39, 0.37, 4.71, 2.5, 1.36, 1.14, 1.00},
+        {16, 128, 256, 1, 0.78, 17.35, 0.73, 5.97, 2.0, 1.40, 0.98, 0.98},
+        {18, 256, 256, 1, 8.68, 23.70, 0.73, 3.89, 0.6, 1.25, 0.98, 1.00},
     };
-    consider(18, 256, 256, 0.02488, 31.4);
-    consider(4, 256, 128, 0.01435, 24.2);
-    consider(5, 128, 128, 0.0107, 8.1);
-    if (split_override > 1 && (!ws_limited || fit_splits(a, ktiles, split_override) > 1))
-        return {best.cfg, split_override};
-    return best;
+    const RingChoice c = pick_ring(kFits, sizeof(kFits) / sizeof(kFits[0]), a, cus, ws_limited, split_override);
+    return {c.id, c.splits};
 }
 
 int64_t w4a16_partial_elems(int64_t rows, int64_t columns, int64_t width, int64_t group) {

@@ -1471,20 +1471,21 @@ hipError_t launch_bn(const W8A8Args& a, hipStream_t stream) {
 // 0 or unset = the shape rule below.
 int w8a8_split_override() { return knob(Knob::W8A8Splits, 0); }
 
-// Split K when 256 x 128 tiles fill at most half of the CUs and K >= 8192,
-// or at most an eighth of them and K >= 4096: K split up to 6 ways, at most
-// one unit per CU, on the 256 x 128 pair ring. The partial sums cost one
-// int32 write and read per element and split, so shorter K, or more tiles,
-// do not pay (MI355X, the reference's shapes: 256 x 4096 x 12288 69 -> 29
-// us, 256 x 3072 x 12288 69 -> 27 us, 512 x 4096 x 12288 69 -> 40 us,
-// 256 x 4096 x 4096 24.7 -> 22.8 us; 512 x 4096 x 4096 26.2 unsplit against
-// 26.6 at best split, 256 x 12288 x 4096 27.8 against 32.5).
+// Split K when 256 x 128 tiles fill at most half of the CUs and K >= 4608, or
+// at most an eighth of them and K >= 4096: K split up to 6 ways, at most one
+// unit per CU, on the 256 x 128 pair ring. The partial sums cost one int32
+// write and read per element and split, so shorter K, or more tiles, do not
+// pay (MI355X, the reference's shapes: 256 x 4096 x 12288 69 -> 29 us, 256 x
+// 3072 x 12288 69 -> 27 us, 512 x 4096 x 12288 69 -> 40 us; 512 x 4096 x 4096
+// 26.2 unsplit against 26.6 at best split, 256 x 12288 x 4096 27.8 against
+// 32.5; between K = 4608 and 8192, rows x K -> N: 503 x 7488 -> 5312 50 -> 35,
+// 160 x 6848 -> 7168 42 -> 26, 301 x 5248 -> 7104 34.1 -> 32.7).
 int w8a8_auto_splits(int64_t rows, int64_t columns, int64_t width, int64_t cus) {
     const int ov = w8a8_split_override();
     if (ov > 1) return ov;
     if (width % 64 != 0 || width < 4096) return 1;
     const int64_t tiles = ((rows + 255) / 256) * ((columns + 127) / 128);
-    if (width >= 8192 ? 2 * tiles > cus : 8 * tiles > cus) return 1;
+    if (width >= 4608 ? 2 * tiles > cus : 8 * tiles > cus) return 1;
     const int64_t want = cus / tiles;
     return (int)(want > 6 ? 6 : want);
 }
@@ -1585,7 +1586,7 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream) {
         if (fit_splits(a, tiles, (int)kt, sp) > 1) {
             // The GEMM and its reduction, us.
             const double m = (double)a.rows / 256.0, mb = 1e-6 * K * (double)a.columns;
-            if (tiles_us < 12.0 + 0.22 * mb + m * (5.0 + 0.09 * mb)) return launch_w8a8_rows(a, tiles_nb, stream);
+            if (0.95 * tiles_us < 13.0 + 0.22 * mb + m * (5.0 + 0.09 * mb)) return launch_w8a8_rows(a, tiles_nb, stream);
             return launch_pair<128>(a, stream, sp);
         }
     }
