@@ -263,9 +263,8 @@ int omni_w8a16_gemm_ws(const uint16_t* x, const int8_t* w, const uint16_t* scale
  * x f16 [rows][width], bias f16 [columns] or NULL, out f16 [rows][columns].
  * width % group == 0 and group % 32 == 0, else OMNI_NOT_HANDLED; x and
  * w_packed 16-byte aligned. One or two rows run the HBM-bound GEMV, up to 32
- * rows a kernel that streams the weights past MFMA (group 128 and an even
- * number of groups; else the skinny MFMA kernel), more rows the fp16-MFMA
- * GEMM. */
+ * rows a kernel that streams the weights past MFMA (group 128; else the
+ * skinny MFMA kernel), more rows the fp16-MFMA GEMM. */
 int omni_w4a16_gemm(const uint16_t* x, const uint8_t* w_packed, const uint16_t* scale_bf16,
                     int64_t group, const uint16_t* bias, int64_t rows, int64_t columns,
                     int64_t width, uint16_t* out, void* stream);

@@ -41,7 +41,7 @@ namespace {
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 // The weights' kind: int8 under int8 activation codes (exact int32 sums),
-// int8, packed int4 (group 128) and f16 under f16 activations.
+// int8, packed int4 (groups of 128) and f16 under f16 activations.
 enum : int { kW8A8, kW8A16, kW4A16, kF16 };
 
 // Activation bytes per weight byte.
@@ -108,11 +108,11 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
     constexpr int RPC = 1024 / TB, XR = 1024 / XTB;  // rows per copy
     constexpr int BM = 16 * MB, BN = 16 * NB;
     constexpr int WC = BN / RPC;                 // weight copies per tile
-    constexpr int SC = WK == kW4A16 ? 1 : 0;     // group scale copies (4 bytes per lane)
+    constexpr int SC = WK == kW4A16 ? TB / 64 : 0;  // group scale copies (one scale per lane)
     constexpr int C = WC + XC + SC;
     constexpr int XROWS = XC * XR;               // activation rows held
     static_assert(XROWS == BM || (MB == 1 && !MT && XROWS < 16 && (XROWS & (XROWS - 1)) == 0), "activation rows");
-    static_assert(WK != kW4A16 || (TB == kInt4Group && BN <= 64), "one dword of group scales per column and tile");
+    static_assert(WK != kW4A16 || BN <= 64, "a lane per column in a scale copy");
     constexpr int kStage = (WC + XC) * 1024 + SC * 256;
     constexpr int kSteps = TB / 64;
     constexpr int kH = WK == kW8A8 ? 1 : x_bytes(WK);  // 16-byte activation pieces per lane and step
@@ -155,11 +155,12 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
     auto w_byte = [&](int c) { return ((lane % (TB / 16)) ^ ((w_row(c) / kW) & kWMask)) * 16; };
     auto x_row = [&](int c) { return c * XR + lane / (XTB / 16); };
     auto x_byte = [&](int c) { return ((lane % (XTB / 16)) ^ ((x_row(c) / kXW) & kXMask)) * 16; };
-    // int4: bytes of a column's group scales (one group per 64 weight bytes).
-    const int srow = wrow / 64 * 2;
+    // int4: a column's group scales (one group of 128 codes per 64 weight bytes).
+    const int groups = wrow / 64;
     // The copies' sources in the unit being issued: wave-uniform bases and
     // per-lane offsets (rows past the matrix repeat the last one).
-    const uint8_t *wbase = nullptr, *xbase = a.x, *sbase = nullptr;
+    const uint8_t *wbase = nullptr, *xbase = a.x;
+    const uint16_t* sbase = nullptr;
     unsigned woff[WC], xoff[XC], soff = 0;
     auto set_unit = [&](int u) {
         const int64_t n0 = unit_n0(u), m0 = unit_m0(u);
@@ -172,8 +173,8 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
 #pragma unroll
         for (int c = 0; c < XC; ++c) xoff[c] = (unsigned)(min(x_row(c), rows) * xrow + x_byte(c));
         if constexpr (SC != 0) {
-            sbase = reinterpret_cast<const uint8_t*>(a.gscale) + n0 * srow;
-            soff = (unsigned)(min(lane, cols) * srow);
+            sbase = a.gscale + n0 * groups;
+            soff = (unsigned)(min(lane, cols) * groups * 2);
         }
     };
     const unsigned st_lds = lds_addr(stages) + wave * (S * kStage);
@@ -193,7 +194,9 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
             else
                 lds_copy16_nt(off, wb, dst + c * 1024);
         }
-        if constexpr (SC != 0) lds_copy4_saddr(soff, sbase + tile * 4, dst + (WC + XC) * 1024);
+#pragma unroll
+        for (int c = 0; c < SC; ++c)
+            lds_copy2_saddr(soff, sbase + min(tile * SC + c, groups - 1), dst + (WC + XC) * 1024 + c * 256);
 #pragma unroll
         for (int c = 0; c < XC; ++c) {
             unsigned off = xoff[c];
@@ -255,7 +258,7 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
             // (16 int8 codes, 32 int4 codes, 8 halves), and the activations of
             // row r at the same k.
             v4u w[kSteps][NB], x[kSteps][MB][kH];
-            u32 sc2[NB];
+            _Float16 sc[kSteps][NB];
 #pragma unroll
             for (int s = 0; s < kSteps; ++s) {
 #pragma unroll
@@ -270,8 +273,11 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
             }
             if constexpr (SC != 0) {
 #pragma unroll
-                for (int j = 0; j < NB; ++j)
-                    sc2[j] = *reinterpret_cast<const u32*>(st + (WC + XC) * 1024 + (j * 16 + r16) * 4);
+                for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j)
+                        sc[s][j] = (_Float16)bf16_to_f32(
+                            *reinterpret_cast<const uint16_t*>(st + (WC + XC) * 1024 + s * 256 + (j * 16 + r16) * 4));
             }
             // Everything is read: the slot takes the next tile while this one
             // is multiplied.
@@ -286,7 +292,10 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
                 for (int s = 0; s < kSteps; ++s)
                     if ((lo + t) * TB + s * 64 + g * 16 >= wrow) {
 #pragma unroll
-                        for (int j = 0; j < NB; ++j) w[s][j] = v4u{0u, 0u, 0u, 0u};
+                        for (int j = 0; j < NB; ++j) {
+                            w[s][j] = v4u{0u, 0u, 0u, 0u};
+                            if constexpr (SC != 0) sc[s][j] = (_Float16)0.0f;
+                        }
 #pragma unroll
                         for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -317,10 +326,9 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
                             i8x4_to_f16x4(wq.z, h[4], h[5]);
                             i8x4_to_f16x4(wq.w, h[6], h[7]);
                         } else {
-                            const _Float16 sc = (_Float16)bf16_to_f32((uint16_t)(s == 0 ? sc2[j] & 0xffffu : sc2[j] >> 16));
                             v2h lo8[8], hi8[8];
-                            i4x16_dequant(wq.x, wq.y, sc, lo8);
-                            i4x16_dequant(wq.z, wq.w, sc, hi8);
+                            i4x16_dequant(wq.x, wq.y, sc[s][j], lo8);
+                            i4x16_dequant(wq.z, wq.w, sc[s][j], hi8);
 #pragma unroll
                             for (int e = 0; e < 8; ++e) h[e] = lo8[e], h[8 + e] = hi8[e];
                         }
@@ -592,16 +600,14 @@ hipError_t launch_w8a16_rows(const W8A16Args& w, hipStream_t st) {
                 : launch_stream_cfg<kW8A16, 4, 1, 8, 3, 4, 64>(a, cus, st);
 }
 
-// Groups of 128, their scales copied two at a time: an even number per
-// column, on a 4-byte boundary. Three to 32 rows, against the GEMV and the
-// skinny kernels: 4 rows of 4096 x 6144 6.8 against 8.7 us, of 3584 x 18944
-// 13.2 against 15.9, 8 of 4096 x 14336 12.2 against 21.6, 16 of 14336 x 4096
-// 16.2 against 28.9, 32 of 3584 x 18944 29.8 against 40.3. The GEMV keeps
-// three and four rows of narrow long-K matrices (4 of 8960 x 1536 7.4
-// against 7.8); one and two rows of K > 32768 are past its limit.
+// Groups of 128. Three to 32 rows, against the GEMV and the skinny kernels:
+// 4 rows of 4096 x 6144 6.8 against 8.7 us, of 3584 x 18944 13.2 against
+// 15.9, 8 of 4096 x 14336 12.2 against 21.6, 16 of 14336 x 4096 16.2 against
+// 28.9, 32 of 3584 x 18944 29.8 against 40.3. The GEMV keeps three and four
+// rows of narrow long-K matrices (4 of 8960 x 1536 7.4 against 7.8); one and
+// two rows of K > 32768 are past its limit.
 bool w4a16_rows_take(const W8A16Args& a) {
-    if (a.rows > 32 || a.group != kInt4Group || a.width % (2 * kInt4Group) != 0 || a.width <= 0 || a.width > kMaxRowBytes ||
-        reinterpret_cast<uintptr_t>(a.gscale) % 4 != 0)
+    if (a.rows > 32 || a.group != kInt4Group || a.width % kInt4Group != 0 || a.width <= 0 || a.width > kMaxRowBytes)
         return false;
     if (a.width > 32768 && a.rows <= 4) return true;
     if (a.rows <= 2) return false;

@@ -920,9 +920,9 @@ hipError_t launch_skinny(const W8A16Args& a, hipStream_t stream) {
 // are exact and the f32 sums stay below 2^13 * sum|x|, so the correction
 // costs ~1e-4 of the result relative and nothing on integer data. A
 // workgroup of T = 64 * ceil(K / 2048) lanes owns R weight rows; every weight
-// load is issued up front. KF > 0 and GF > 0 build the kernel for K == KF,
-// a multiple of 2048 (every lane then owns one chunk), and group == GF: no
-// clamp, and the scale index without a 64-bit division.
+// load is issued up front. GF > 0 builds the kernel for group == GF: the scale
+// index without a 64-bit division. KF > 0 (with GF) builds it for K == KF, a
+// multiple of 2048 (every lane then owns one chunk): no clamp.
 // TEAMS > 1 (K == KF builds only): the workgroup holds TEAMS teams of
 // T = KF / 32 lanes, team t taking the R * B rows after team t - 1's, so a
 // 2-wave team's rows share a workgroup (and its launch) with the next team's
@@ -933,7 +933,7 @@ __global__ __launch_bounds__(KF > 0 ? KF / 32 * TEAMS : 1024) void w4a16_gemv_ke
     constexpr int V = R * MR;
     constexpr int RB = R * B;  // rows per team: B batches of R
     static_assert((V & (V - 1)) == 0 && V <= 64, "power-of-two partial count");
-    static_assert(KF % 2048 == 0 && (KF == 0) == (GF == 0), "KF: a multiple of 2048, with GF");
+    static_assert(KF % 2048 == 0 && (KF == 0 || GF > 0), "KF: a multiple of 2048, with GF");
     static_assert(TEAMS == 1 || (KF > 0 && KF / 32 * TEAMS <= 1024), "teams: K == KF builds within 1024 lanes");
     __shared__ float s_part[16][B * V];
     typedef unsigned v4u __attribute__((ext_vector_type(4)));
@@ -1362,8 +1362,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 1) void w8a16_mfma_kernel(W
 // the group scale in f16), four codes at a time spread over the MFMA slots
 // of the pair before the one that uses them, so the conversion overlaps the
 // MFMAs. The scales ride in the ring too: behind each stage's
-// rows, the aligned bf16 pair holding the tile's group for every column (one
-// 4-byte-per-lane copy per wave per K tile, 64 columns each).
+// rows, the bf16 scale of the tile's group for every column, a dword each (one
+// 2-byte-per-lane copy per wave per K tile, 64 columns each).
 template <int BM, int BN, int WB = 8, int WMW = 2, int S = 3, int KP = 2, int OCC = 1, bool SK = false, int NW = 4>
 __global__ __launch_bounds__(64 * NW, OCC) void w8a16_ring_kernel(W8A16Args a, int splits) {
     static_assert(S == 2 || S == 3, "2 or 3 stages");
@@ -1516,7 +1516,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void w8a16_ring_kernel(W8A16Args a, i
             ktiles = min(kts, ktiles_all - kbase);
         }
     };
-    // int4: group of K tile kk (a scale pair holds groups 2i, 2i + 1).
+    // int4: K tiles per group.
     const int gdiv = WB == 4 ? (int)(a.group / 64) : 1;
     auto copy_one = [&](int kt, int s, int j) {
         const int64_t kk = kbase + min(kt, ktiles - 1);
@@ -1526,11 +1526,9 @@ __global__ __launch_bounds__(64 * NW, OCC) void w8a16_ring_kernel(W8A16Args a, i
                                    : reinterpret_cast<const uint8_t*>(a.w) + kk * kWBytes;
         lds_copy16_saddr(voff[j], base, stage_lds[s] + c * 1024);
         if constexpr (WB == 4) {
-            if (j == kCpw - 1) {
-                const int g = (int)kk / gdiv;
-                lds_copy4_saddr(voff_sc, a.gscale + (g & ~1),
+            if (j == kCpw - 1)
+                lds_copy2_saddr(voff_sc, a.gscale + (int)kk / gdiv,
                                 stage_lds[s] + kScOff + (wave % (BN / 64)) * 256);
-            }
         }
     };
     auto copy_tile = [&](int kt, int s) {
@@ -1565,11 +1563,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void w8a16_ring_kernel(W8A16Args a, i
                 } else {
                     const uint2 w2 = *reinterpret_cast<const uint2*>(stage(s) + offB4(p) + idx * 16 * 64);
                     xb[idx][0] = v4i{(int)w2.x, (int)w2.y, 0, 0};
-                    if (p == 0) {
-                        const int g = (int)(kbase + kt) / gdiv;
-                        sc[idx] = *reinterpret_cast<const uint16_t*>(stage(s) + kScOff +
-                                                                     (wn * WN + 32 * idx + fr) * 4 + (g & 1) * 2);
-                    }
+                    if (p == 0)
+                        sc[idx] = *reinterpret_cast<const uint16_t*>(stage(s) + kScOff + (wn * WN + 32 * idx + fr) * 4);
                 }
             } else {
                 const int i = idx - FN;
@@ -2149,12 +2144,13 @@ hipError_t launch_w4a16_gemv(const W8A16Args& a, hipStream_t stream) {
     // OMNI_W4A16_GEMV=<r><b> pins r rows per batch and b batches per
     // workgroup (tuning aid); unset: the measured choice below.
     int cfg = knob(Knob::W4A16Gemv, 0);
-    // Measured on MI355X: 4 rows per workgroup from 4 MB of codes (7.6 us
-    // at 4096 x 14336), two batches of 4 from 64 MB (43 us at the 128256-row
-    // vocabulary head), 2 rows below 4 MB. With 2-4 activation rows, 8 rows
-    // per workgroup from 16 MB (4096 x 14336, 4 rows: 13.4 against 15.0 us;
-    // 14336 x 4096, 3 rows: 13.0 against 14.5; 4096 x 4096 stays on 4 rows,
-    // 6.3 against 7.9).
+    // Measured on MI355X: 2 rows per workgroup below 4 MB of codes, 4 rows from
+    // there (7.6 us at 4096 x 14336), two batches of 4 from 24 MB (2944 x 25088
+    // 10.4 us against 11.6, 18944 x 3584 10.1 against 10.6; the 128256-row
+    // vocabulary head 43), with 3 or 4 activation rows from 64 MB. With 2-4
+    // activation rows, 8 rows per workgroup from 16 MB (4096 x 14336, 4 rows:
+    // 13.4 against 15.0 us; 14336 x 4096, 3 rows: 13.0 against 14.5; 4096 x
+    // 4096 stays on 4 rows, 6.3 against 7.9).
     const int64_t code_bytes = a.columns * a.width / 2;
     // One row at K = 4096, group 128, from 4 MB of codes: two 128-lane teams
     // of 8 rows per workgroup (MI355X, weights rotated past the MALL, against
@@ -2166,7 +2162,7 @@ hipError_t launch_w4a16_gemv(const W8A16Args& a, hipStream_t stream) {
         return hipGetLastError();
     }
     if (cfg == 0) {
-        if (code_bytes >= (64 << 20)) cfg = 42;
+        if (code_bytes >= (a.rows <= 2 ? 24 << 20 : 64 << 20)) cfg = 42;
         else if (a.rows >= 2 && code_bytes >= (16 << 20)) cfg = 81;
         else cfg = code_bytes >= (4 << 20) ? 41 : 21;
     }
@@ -2184,6 +2180,14 @@ hipError_t launch_w4a16_gemv(const W8A16Args& a, hipStream_t stream) {
                 hipLaunchKernelGGL((w4a16_gemv_kernel<1, R, B, 14336, 128>), grid, block, 0, stream, a);
                 return hipGetLastError();
             }
+        }
+        if (a.group == 128) {
+            switch (a.rows) {
+                case 1: hipLaunchKernelGGL((w4a16_gemv_kernel<1, R, B, 0, 128>), grid, block, 0, stream, a); break;
+                case 2: hipLaunchKernelGGL((w4a16_gemv_kernel<2, R, B, 0, 128>), grid, block, 0, stream, a); break;
+                default: hipLaunchKernelGGL((w4a16_gemv_kernel<4, R, B, 0, 128>), grid, block, 0, stream, a); break;
+            }
+            return hipGetLastError();
         }
         switch (a.rows) {
             case 1: hipLaunchKernelGGL((w4a16_gemv_kernel<1, R, B>), grid, block, 0, stream, a); break;
@@ -2250,7 +2254,7 @@ hipError_t launch_w4a16_skinny(const W8A16Args& a, hipStream_t stream) {
 // rings 4 / 5 / 6 = 256 x 128 / 128 x 128 / 256 x 256, 10 = 128 x 128 at
 // two workgroups per CU, 16 / 17 / 18 = eight-wave 128 x 256 / 256 x 256
 // (waves 64 x 128) / 256 x 256 (waves 128 x 64) (rings: K % 64 == 0, group
-// % 64 == 0, K / group even, scales 4-byte aligned); OMNI_W4A16_SPLITS=<n>
+// % 64 == 0); OMNI_W4A16_SPLITS=<n>
 // adds n-way split K to a pinned ring when the call brings a workspace.
 // Both are tuning knobs (omni::knob).
 struct W4Plan {
@@ -2258,12 +2262,7 @@ struct W4Plan {
     int splits;  // K splits (> 1 needs a workspace)
 };
 
-// (the ring copies a column's scales as aligned bf16 pairs: an even count
-// per row, from a 4-byte aligned scale array)
-bool w4_ring_ok(const W8A16Args& a) {
-    return ring16_fits(a) && a.group % 64 == 0 && (a.width / a.group) % 2 == 0 &&
-           reinterpret_cast<uintptr_t>(a.gscale) % 4 == 0;
-}
+bool w4_ring_ok(const W8A16Args& a) { return ring16_fits(a) && a.group % 64 == 0; }
 
 W4Plan plan_w4a16(const W8A16Args& a, int cus, bool ws_limited) {
     const int split_override = knob(Knob::W4A16Splits, 0);

@@ -107,7 +107,8 @@ def test_w8a16_stream(rows, width, columns):
 @pytest.mark.parametrize("rows,width,columns", [
     (1, 33024, 20), (3, 256, 5), (4, 2304, 33), (4, 4352, 2050), (3, 4352, 4100), (4, 512, 4100), (4, 256, 20000),
     (5, 256, 15), (8, 1792, 100), (7, 768, 4100), (9, 3328, 17), (16, 256, 64), (13, 1280, 4097), (17, 512, 31),
-    (32, 2816, 70), (29, 768, 4129), (6, 256, 131100)])
+    (32, 2816, 70), (29, 768, 4129), (6, 256, 131100), (5, 128, 33), (8, 1152, 100), (16, 2944, 4099), (3, 4224, 2051),
+    (32, 1408, 65), (17, 384, 4130)])
 def test_w4a16_stream(oracle, rows, width, columns):
     rng = np.random.default_rng(rows + 5 * width + columns)
     x = rng.standard_normal((rows, width)).astype(np.float16)
