@@ -1998,16 +1998,18 @@ hipError_t launch_w8a16_skinny(const W8A16Args& a, hipStream_t stream) { return 
 // 64 x 128, 9 = ring 256 x 192, 10 = ring 128 x 128 two workgroups per CU,
 // 11 / 12 = ring 64 x 128 two / three per CU, 16 / 17 / 18 = ring 128 x 256 /
 // 256 x 256 (waves 64 x 128) / 256 x 256 (waves 128 x 64) with eight waves,
-// 19 / 20 / 21 = ring 128 x 320 / 64 x 192 / 128 x 192 (rings: K % 64 == 0
-// only). OMNI_W8A16_SPLITS=<n>
-// adds n-way split K to a pinned ring (or to the shape rule's choice) when
-// the call brings a workspace. Both are tuning knobs (omni::knob).
+// 19 / 20 / 21 = ring 128 x 320 / 64 x 192 / 128 x 192, 22 = ring 192 x 256
+// with eight waves (rings: K % 64 == 0 only). OMNI_W8A16_SPLITS=<n> adds n-way
+// split K to a pinned ring (or to the shape rule's choice) when the call
+// brings a workspace. Both are tuning knobs (omni::knob).
 int w8a16_tile_override() { return knob(Knob::W8A16Tile, 0); }
 
 // One ring kernel's time in us, fitted to measurements: units (tiles, times
 // the splits of K) run in rounds of occ per CU, a full round takes a + b K /
-// splits / 1000, a partial last one with fill f p + (1 - p) f of that, a launch
-// t0, and a split's reduction r0 + r1 us per million of its partial sums.
+// splits / 1000, a partial last one p + (1 - p) f of that (f: its fill; with
+// two or three workgroups per CU the busiest CU's share of them past the
+// first), a launch t0, and a split's reduction r0 + r1 us per million of its
+// partial sums.
 // unsplit and split weigh the estimate where its error has a sign. r0 = 0: not
 // split.
 struct RingFit {
@@ -2032,7 +2034,9 @@ RingChoice pick_ring(const RingFit* fits, size_t count, const W8A16Args& a, int 
         auto time = [&](int sp) {
             const int64_t units = tiles * sp, slots = (int64_t)cus * f.occ;
             const int64_t full = units / slots, rem = units % slots;
-            const double rounds = (double)full + (rem ? f.p + (1.0 - f.p) * (double)rem / (double)slots : 0.0);
+            const double fill = f.occ == 1 ? (double)rem / (double)slots
+                                           : (double)((rem + cus - 1) / cus - 1) / (double)(f.occ - 1);
+            const double rounds = (double)full + (rem ? f.p + (1.0 - f.p) * fill : 0.0);
             double t = f.t0 + rounds * (f.a + 1e-3 * f.b * (double)a.width / sp);
             if (sp == 1) return t * f.unsplit;
             return (t + f.r0 + 1e-6 * f.r1 * sp * (double)a.rows * (double)a.columns) * f.split;
@@ -2066,7 +2070,7 @@ W16Plan plan_w8a16(const W8A16Args& a, int cus, bool ws_limited) {
     const int split_override = knob(Knob::W8A16Splits, 0);
     const bool ring_ok = ring16_fits(a);
     const int ov = w8a16_tile_override();
-    if (ov == 1 || ov == 2 || (ov >= 4 && ov <= 12 && ring_ok) || (ov >= 16 && ov <= 21 && ring_ok))
+    if (ov == 1 || ov == 2 || (ov >= 4 && ov <= 12 && ring_ok) || (ov >= 16 && ov <= 22 && ring_ok))
         return {ov, ov >= 4 && split_override > 1 ? split_override : 1};
     if (!ring_ok) {
         const int64_t big_tiles = ((a.rows + 127) / 128) * ((a.columns + 127) / 128);
@@ -2074,22 +2078,24 @@ W16Plan plan_w8a16(const W8A16Args& a, int cus, bool ws_limited) {
     }
     // MI355X fits over 150 shapes (65 to 4352 rows, K 1024 ... 14336, N 1024 ...
     // 18944, every ring and split; median error 2-6 %). The choice by them is
-    // within 2 % of the fastest on average, where the rules it replaces (one
-    // model for the one-per-CU rings, hand-set lines for splits and small
-    // tiles) were 9 % off: 582 x 7680 -> 3264 41 us against 69 (128 x 192 tiles
-    // split three ways), 109 x 3968 -> 2112 14 against 22; config 5's gate/up
-    // (128 x 320 tiles) and down (128 x 192 split four ways) are as before.
+    // within 1 % of the fastest on average, where one model for the
+    // one-per-CU rings and hand-set lines for splits and small tiles were 10 %
+    // off: 582 x 7680 -> 3264 41 us against 69 (128 x 192 tiles split three
+    // ways), 109 x 3968 -> 2112 14 against 22. 192 x 256 tiles fill the rounds
+    // that 128 x 320 and 256 x 256 leave ragged: 2550 x 1152 -> 8064 55 us
+    // against 63, 159 x 11008 -> 17920 83 (split three ways) against 107.
     static constexpr RingFit kFits[] = {
-        {5, 128, 128, 1, 4.67, 7.53, 0.69, 1.97, 0.0, 0.00, 0.98, 1.00},
-        {8, 64, 128, 1, 2.63, 5.39, 0.83, 2.13, 0.0, 0.00, 1.10, 1.00},
-        {9, 256, 192, 1, 10.32, 17.21, 0.73, 4.28, 1.3, 0.81, 1.00, 0.96},
-        {10, 128, 128, 2, 5.25, 14.94, 0.30, 3.45, 2.8, 0.87, 1.02, 1.04},
-        {12, 64, 128, 3, 4.47, 14.73, 0.24, 2.81, 2.8, 0.78, 0.98, 1.00},
-        {16, 128, 256, 1, 5.66, 13.01, 0.65, 2.56, 2.7, 0.82, 1.00, 1.00},
-        {18, 256, 256, 1, 15.52, 20.34, 0.67, 0.00, 1.8, 0.81, 1.00, 1.06},
+        {5, 128, 128, 1, 4.67, 7.53, 0.69, 1.97, 0.0, 0.00, 1.08, 1.00},
+        {8, 64, 128, 1, 2.63, 5.39, 0.83, 2.13, 0.0, 0.00, 1.00, 1.00},
+        {9, 256, 192, 1, 10.32, 17.21, 0.73, 4.28, 1.3, 0.81, 1.00, 1.00},
+        {10, 128, 128, 2, 0.71, 13.57, 0.45, 5.10, 2.4, 1.53, 1.14, 1.00},
+        {12, 64, 128, 3, 4.21, 13.31, 0.36, 2.48, 3.1, 0.95, 0.94, 1.02},
+        {16, 128, 256, 1, 5.66, 13.01, 0.65, 2.56, 2.7, 0.82, 0.96, 1.00},
+        {18, 256, 256, 1, 15.52, 20.34, 0.67, 0.00, 1.8, 0.81, 0.92, 1.00},
         {19, 128, 320, 1, 10.28, 15.39, 0.73, 1.80, 2.3, 0.75, 1.00, 1.00},
-        {20, 64, 192, 1, 3.95, 7.29, 0.83, 2.11, 0.0, 0.00, 1.00, 1.00},
-        {21, 128, 192, 1, 5.34, 9.82, 0.67, 3.71, 2.4, 0.89, 1.00, 1.06},
+        {20, 64, 192, 1, 3.95, 7.29, 0.83, 2.11, 0.0, 0.00, 1.02, 1.00},
+        {21, 128, 192, 1, 5.34, 9.82, 0.67, 3.71, 2.4, 0.89, 1.00, 1.00},
+        {22, 192, 256, 1, 7.80, 16.42, 0.63, 2.46, 2.2, 0.81, 0.92, 1.02},
     };
     const RingChoice c = pick_ring(kFits, sizeof(kFits) / sizeof(kFits[0]), a, cus, ws_limited, split_override);
     return {c.id, c.splits};
@@ -2132,6 +2138,7 @@ hipError_t launch_w8a16_mfma(const W8A16Args& a, hipStream_t stream) {
         case 19: return launch_ring16_cfg<128, 320>(a, stream, sp);
         case 20: return launch_ring16_cfg<64, 192>(a, stream, sp);
         case 21: return launch_ring16_cfg<128, 192>(a, stream, sp);
+        case 22: return launch_ring16_cfg<192, 256, 8, 2, 3, 2, 1, 8>(a, stream, sp);
         default: return launch_ring16_cfg<64, 128, 8, 2, 3, 2, 3>(a, stream, sp);
     }
 }
@@ -2253,10 +2260,10 @@ hipError_t launch_w4a16_skinny(const W8A16Args& a, hipStream_t stream) {
 // 1 / 2 = tiled 128 x 128 / 64 x 64 (codes dequantized through registers),
 // rings 4 / 5 / 6 = 256 x 128 / 128 x 128 / 256 x 256, 10 = 128 x 128 at
 // two workgroups per CU, 16 / 17 / 18 = eight-wave 128 x 256 / 256 x 256
-// (waves 64 x 128) / 256 x 256 (waves 128 x 64) (rings: K % 64 == 0, group
-// % 64 == 0); OMNI_W4A16_SPLITS=<n>
-// adds n-way split K to a pinned ring when the call brings a workspace.
-// Both are tuning knobs (omni::knob).
+// (waves 64 x 128) / 256 x 256 (waves 128 x 64) / 22 = 192 x 256 (rings:
+// K % 64 == 0, group % 64 == 0); OMNI_W4A16_SPLITS=<n> adds n-way split K to a
+// pinned ring when the call brings a workspace. Both are tuning knobs
+// (omni::knob).
 struct W4Plan {
     int cfg;     // tile id as above
     int splits;  // K splits (> 1 needs a workspace)
@@ -2269,7 +2276,7 @@ W4Plan plan_w4a16(const W8A16Args& a, int cus, bool ws_limited) {
     const int t = knob(Knob::W4A16Tile, 0);
     const bool ring_ok = w4_ring_ok(a);
     if (t == 1 || t == 2) return {t, 1};
-    if (ring_ok && (t == 4 || t == 5 || t == 6 || t == 10 || (t >= 16 && t <= 18)))
+    if (ring_ok && (t == 4 || t == 5 || t == 6 || t == 10 || (t >= 16 && t <= 18) || t == 22))
         return {t, split_override > 1 ? split_override : 1};
     if (!ring_ok) {
         const int64_t big_tiles = ((a.rows + 127) / 128) * ((a.columns + 127) / 128);
@@ -2277,16 +2284,17 @@ W4Plan plan_w4a16(const W8A16Args& a, int cus, bool ws_limited) {
     }
     // MI355X fits over 130 shapes (33 to 4352 rows, K 1024 ... 14336, N 1024 ...
     // 18944, every ring and split; median error 3-6 %). The choice by them is
-    // within 1 % of the fastest on average and 4 % slower than before at worst,
-    // where the three rings it knew, split only from K = 4096 on, were 11 % off:
-    // 67 x 3328 -> 1664 16 us against 35, 191 x 2816 -> 1280 16 against 30 (128
-    // x 128 tiles two per CU, split four ways).
+    // within 1 % of the fastest on average, where three rings, split only from
+    // K = 4096 on, were 13 % off: 67 x 3328 -> 1664 16 us against 35, 191 x
+    // 2816 -> 1280 16 against 30 (128 x 128 tiles two per CU, split four ways);
+    // 192 x 256 tiles 916 x 2560 -> 8704 53 us against 63 in 256 x 256.
     static constexpr RingFit kFits[] = {
-        {4, 256, 128, 1, 4.01, 15.18, 0.72, 7.28, 0.7, 1.24, 1.04, 0.98},
-        {5, 128, 128, 1, 1.65, 10.44, 0.77, 5.00, 2.2, 1.32, 1.02, 1.00},
-        {10, 128, 128, 2, 1.50, 19.39, 0.37, 4.71, 2.5, 1.36, 1.14, 1.00},
-        {16, 128, 256, 1, 0.78, 17.35, 0.73, 5.97, 2.0, 1.40, 0.98, 0.98},
-        {18, 256, 256, 1, 8.68, 23.70, 0.73, 3.89, 0.6, 1.25, 0.98, 1.00},
+        {4, 256, 128, 1, 4.01, 15.18, 0.72, 7.28, 0.7, 1.24, 1.02, 0.96},
+        {5, 128, 128, 1, 1.65, 10.44, 0.77, 5.00, 2.2, 1.32, 0.98, 1.00},
+        {10, 128, 128, 2, 0.00, 16.60, 0.56, 5.63, 1.8, 1.78, 1.06, 1.00},
+        {16, 128, 256, 1, 0.78, 17.35, 0.73, 5.97, 2.0, 1.40, 0.96, 0.98},
+        {18, 256, 256, 1, 8.68, 23.70, 0.73, 3.89, 0.6, 1.25, 1.00, 1.06},
+        {22, 192, 256, 1, 2.84, 21.39, 0.65, 5.12, 2.4, 1.22, 1.00, 0.92},
     };
     const RingChoice c = pick_ring(kFits, sizeof(kFits) / sizeof(kFits[0]), a, cus, ws_limited, split_override);
     return {c.id, c.splits};
@@ -2316,6 +2324,7 @@ hipError_t launch_w4a16_mfma(const W8A16Args& a, hipStream_t stream) {
         case 10: return launch_ring16_cfg<128, 128, 4, 2, 3, 2, 2>(a, stream, sp);
         case 16: return launch_ring16_cfg<128, 256, 4, 2, 3, 2, 1, 8>(a, stream, sp);
         case 17: return launch_ring16_cfg<256, 256, 4, 4, 3, 2, 1, 8>(a, stream, sp);
+        case 22: return launch_ring16_cfg<192, 256, 4, 2, 3, 2, 1, 8>(a, stream, sp);
         default: return launch_ring16_cfg<256, 256, 4, 2, 3, 2, 1, 8>(a, stream, sp);
     }
 }

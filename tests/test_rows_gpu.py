@@ -129,3 +129,25 @@ def test_f16_stream(rows, width, columns):
     x = rng.standard_normal((rows, width)).astype(np.float16)
     w = (rng.standard_normal((columns, width)) * 0.05).astype(np.float16)
     close(f16.depth_try_linear(dev(x), dev(w).t()), x.astype(np.float64) @ w.T.astype(np.float64))
+
+
+# The 192 x 256 ring: both sides of a tile's edge in rows and columns, one and
+# several K tiles per split, whole and split three ways.
+@pytest.mark.parametrize("splits", ["1", "3"])
+@pytest.mark.parametrize("rows,width,columns", [
+    (1, 128, 255), (191, 384, 257), (192, 512, 256), (193, 1408, 300), (385, 640, 770), (500, 2944, 513)])
+def test_ring_192(rows, width, columns, splits, knobs):
+    for name in ("OMNI_W8A16", "OMNI_W4A16"):
+        knobs.set(name + "_TILE", "22")
+        knobs.set(name + "_SPLITS", splits)
+    rng = np.random.default_rng(rows + width + columns)
+    x = rng.standard_normal((rows, width)).astype(np.float16)
+    w = rng.integers(-128, 128, (columns, width), dtype=np.int8)
+    scale = rng.uniform(0.002, 0.02, columns).astype(np.float16)
+    exact = (x.astype(np.float64) @ w.T.astype(np.float64)) * scale.astype(np.float64)
+    close(oi.w8a16_linear(dev(x), dev(w), dev(scale)), exact)
+    packed = w.view(np.uint8)[:, :width // 2]
+    gscale = torch.from_numpy(rng.uniform(0.002, 0.02, (columns, width // 128)).astype(np.float32)).bfloat16()
+    q = np.stack((packed & 15, packed >> 4), -1).reshape(columns, width).astype(np.float64) - 8
+    exact = x.astype(np.float64) @ (q * np.repeat(gscale.double().numpy(), 128, 1)).T
+    close(oi.w4a16_linear(dev(x), dev(packed), gscale.cuda()), exact)
