@@ -258,7 +258,7 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
             // (16 int8 codes, 32 int4 codes, 8 halves), and the activations of
             // row r at the same k.
             v4u w[kSteps][NB], x[kSteps][MB][kH];
-            _Float16 sc[kSteps][NB];
+            float sc[kSteps][NB];
 #pragma unroll
             for (int s = 0; s < kSteps; ++s) {
 #pragma unroll
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
                 for (int s = 0; s < kSteps; ++s)
 #pragma unroll
                     for (int j = 0; j < NB; ++j)
-                        sc[s][j] = (_Float16)bf16_to_f32(
+                        sc[s][j] = bf16_to_f32(
                             *reinterpret_cast<const uint16_t*>(st + (WC + XC) * 1024 + s * 256 + (j * 16 + r16) * 4));
             }
             // Everything is read: the slot takes the next tile while this one
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
 #pragma unroll
                         for (int j = 0; j < NB; ++j) {
                             w[s][j] = v4u{0u, 0u, 0u, 0u};
-                            if constexpr (SC != 0) sc[s][j] = (_Float16)0.0f;
+                            if constexpr (SC != 0) sc[s][j] = 0.0f;
                         }
 #pragma unroll
                         for (int i = 0; i < MB; ++i)
@@ -326,25 +326,48 @@ __global__ __launch_bounds__(64 * KW, KW / 4) void rows_stream_kernel(RowsArgs a
                             i8x4_to_f16x4(wq.z, h[4], h[5]);
                             i8x4_to_f16x4(wq.w, h[6], h[7]);
                         } else {
-                            v2h lo8[8], hi8[8];
-                            i4x16_dequant(wq.x, wq.y, sc[s][j], lo8);
-                            i4x16_dequant(wq.z, wq.w, sc[s][j], hi8);
+                            const unsigned word[4] = {wq.x, wq.y, wq.z, wq.w};
 #pragma unroll
-                            for (int e = 0; e < 8; ++e) h[e] = lo8[e], h[8 + e] = hi8[e];
+                            for (int q = 0; q < 4; ++q) {
+                                v2h h4[4];
+                                i4x8_to_f16x8(word[q], h4);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) h[4 * q + e] = h4[e];
+                            }
                         }
 #pragma unroll
                         for (int q = 0; q < kH; ++q)
                             b[j][q] = v8h{h[4 * q][0],     h[4 * q][1],     h[4 * q + 1][0], h[4 * q + 1][1],
                                           h[4 * q + 2][0], h[4 * q + 2][1], h[4 * q + 3][0], h[4 * q + 3][1]};
                     }
+                    // int4: the step's 64 bytes are one group, whose sum takes its
+                    // scale in f32, four FMAs per 16 x 16 block (a lane's sums are of
+                    // one column). Scaling the codes in f16 first took 16 packed
+                    // multiplies per column block and lost scales outside f16's
+                    // normal range (3 rows of 4096 x 14336 10.6 against 11.4 us, 8 of
+                    // 3584 x 18944 15.1 against 15.9, 16 17.5 against 18.2; 32 rows
+                    // even).
+                    Acc group[NB][MB];
 #pragma unroll
                     for (int q = 0; q < kH; ++q)
 #pragma unroll
                         for (int i = 0; i < MB; ++i)
 #pragma unroll
+                            for (int j = 0; j < NB; ++j) {
+                                const bool first_of = WK == kW4A16 && q == 0;
+                                Acc& to = WK == kW4A16 ? group[j][i] : acc[j][i];
+                                to = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, x[s][i][q]),
+                                                                           b[j][q], first_of ? Acc{} : to, 0, 0, 0);
+                            }
+                    if constexpr (WK == kW4A16) {
+#pragma unroll
+                        for (int i = 0; i < MB; ++i)
+#pragma unroll
                             for (int j = 0; j < NB; ++j)
-                                acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, x[s][i][q]),
-                                                                                  b[j][q], acc[j][i], 0, 0, 0);
+#pragma unroll
+                                for (int r = 0; r < 4; ++r)
+                                    acc[j][i][r] = __builtin_fmaf(group[j][i][r], sc[s][j], acc[j][i][r]);
+                    }
                 }
             }
             ++done;

@@ -121,6 +121,26 @@ def test_w4a16_stream(oracle, rows, width, columns):
     close(oi.w4a16_linear(dev(x), dev(packed), scale.cuda(), dev(bias)), exact + bias.astype(np.float64))
 
 
+# Group scales outside f16's normal range enter in f32: the result is off by its
+# rounding to f16 (half a unit, 2^-11 of the value or 2^-25) and by the f32 sums'
+# (2^-24 of the absolute sum for each of `width` additions), no more.
+@pytest.mark.parametrize("low,high", [(1e-6, 5e-5), (8192.0, 65536.0)])
+@pytest.mark.parametrize("rows,width,columns", [
+    (3, 256, 2100), (4, 640, 33), (8, 384, 100), (16, 512, 4200), (32, 128, 70)])
+def test_w4a16_stream_scales(rows, width, columns, low, high):
+    rng = np.random.default_rng(rows + width + columns)
+    x = (rng.standard_normal((rows, width)) * (1.0 if high < 1 else 2e-3)).astype(np.float16)
+    packed = rng.integers(0, 256, (columns, width // 2), dtype=np.uint8)
+    scale = torch.from_numpy(rng.uniform(low, high, (columns, width // 128)).astype(np.float32)).bfloat16()
+    q = np.stack((packed & 15, packed >> 4), -1).reshape(columns, width).astype(np.float64) - 8
+    w = q * np.repeat(scale.double().numpy(), 128, 1)
+    exact, total = x.astype(np.float64) @ w.T, np.abs(x.astype(np.float64)) @ np.abs(w).T
+    got = host(oi.w4a16_linear(dev(x), dev(packed), scale.cuda())).astype(np.float64)
+    bound = np.abs(exact) * 2.0**-11 + 2.0**-25 + width * 2.0**-24 * total
+    fits = np.abs(exact) < 65504 * (1 - 2.0**-10)
+    assert fits.any() and (np.abs(got - exact) <= bound)[fits].all()
+
+
 @pytest.mark.parametrize("rows,width,columns", [
     (5, 32, 9), (8, 160, 100), (9, 1056, 33), (16, 8192, 17), (17, 96, 64), (32, 544, 40), (33, 64, 31),
     (48, 1120, 70), (49, 32, 16), (64, 2080, 95)])
