@@ -262,15 +262,16 @@ int omni_w8a16_gemm_ws(const uint16_t* x, const int8_t* w, const uint16_t* scale
  *   out[m][n] = f16(sum_k x[m][k] * (q[n][k] * scale[n][k / group]) + bias[n])
  * x f16 [rows][width], bias f16 [columns] or NULL, out f16 [rows][columns].
  * width % group == 0 and group % 32 == 0, else OMNI_NOT_HANDLED; x and
- * w_packed 16-byte aligned. One or two rows run the HBM-bound GEMV, up to 32
+ * w_packed 16-byte aligned. One or two rows run the HBM-bound GEMV, up to 64
  * rows a kernel that streams the weights past MFMA (group 128; else the
- * skinny MFMA kernel), more rows the fp16-MFMA GEMM. */
+ * skinny MFMA kernel), more rows (and from 49 on, wide matrices) the
+ * fp16-MFMA GEMM. */
 int omni_w4a16_gemm(const uint16_t* x, const uint8_t* w_packed, const uint16_t* scale_bf16,
                     int64_t group, const uint16_t* bias, int64_t rows, int64_t columns,
                     int64_t width, uint16_t* out, void* stream);
 
 /* Bytes of workspace omni_w4a16_gemm_ws uses at most for this shape on the
- * current device (calls of up to 32 rows may run without): split-K partial sums (f32 [splits][rows][columns]) for the shapes
+ * current device (calls of few rows may run without): split-K partial sums (f32 [splits][rows][columns]) for the shapes
  * that split (GEMM shapes, and 5..16 rows over long K and many columns); 0
  * when the shape does not split. No counterpart in the reference: it
  * serves omni_w4a16_gemm_ws. */

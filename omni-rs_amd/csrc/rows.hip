@@ -623,18 +623,27 @@ hipError_t launch_w8a16_rows(const W8A16Args& w, hipStream_t st) {
                 : launch_stream_cfg<kW8A16, 4, 1, 8, 3, 4, 64>(a, cus, st);
 }
 
-// Groups of 128. Three to 32 rows, against the GEMV and the skinny kernels:
+// Groups of 128. Three to 64 rows, against the GEMV, the skinny kernels and the
+// GEMM:
 // 4 rows of 4096 x 6144 6.8 against 8.7 us, of 3584 x 18944 13.2 against
 // 15.9, 8 of 4096 x 14336 12.2 against 21.6, 16 of 14336 x 4096 16.2 against
 // 28.9, 32 of 3584 x 18944 29.8 against 40.3. The GEMV keeps three and four
 // rows of narrow long-K matrices (4 of 8960 x 1536 7.4 against 7.8); one and
-// two rows of K > 32768 are past its limit.
+// two rows of K > 32768 are past its limit. 48 rows of 4096 x 6144 12.5 against
+// 32.2 us, of 8192 x 28672 80 against 93; from 49 rows on, in blocks of 16
+// columns (64 of 8960 x 1536 21.2 against 37.9, of 2048 x 8192 12.6 against
+// 18.3, of 4096 x 6144 19.4 against 20.6), the GEMM keeps what is wide and large
+// (64 of 4096 x 14336 36.0 against 30.0) or very wide (of 1024 x 18944 16.4
+// against 14.8).
 bool w4a16_rows_take(const W8A16Args& a) {
-    if (a.rows > 32 || a.group != kInt4Group || a.width % kInt4Group != 0 || a.width <= 0 || a.width > kMaxRowBytes)
+    if (a.rows > 64 || a.group != kInt4Group || a.width % kInt4Group != 0 || a.width <= 0 || a.width > kMaxRowBytes)
         return false;
     if (a.width > 32768 && a.rows <= 4) return true;
     if (a.rows <= 2) return false;
-    return a.rows > 4 || a.columns > 2048 || a.width <= 4096;
+    if (a.rows <= 4) return a.columns > 2048 || a.width <= 4096;
+    const int64_t cus = num_cus();
+    return a.rows <= 48 || !is_wide(a.columns, cus) ||
+           (a.columns <= 40 * cus && (double)a.columns * (double)a.width <= 26e6);
 }
 
 hipError_t launch_w4a16_rows(const W8A16Args& w, hipStream_t st) {
@@ -656,8 +665,16 @@ hipError_t launch_w4a16_rows(const W8A16Args& w, hipStream_t st) {
     if (w.rows <= 16)
         return wide ? launch_stream_cfg<kW4A16, 1, 2, 8, 2, 4, 128>(a, cus, st)
                     : launch_stream_cfg<kW4A16, 1, 1, 8, 3, 4, 128>(a, cus, st);
-    return wide ? launch_stream_cfg<kW4A16, 2, 2, 16, 1, 4, 128>(a, cus, st)
-                : launch_stream_cfg<kW4A16, 2, 1, 16, 1, 4, 128>(a, cus, st);
+    // One 128-byte tile, not three of 64 (32 rows of 4096 x 14336 17.6 against
+    // 18.7, of 8960 x 1536 13.0 against 13.6; 17 to 24 rows even).
+    if (w.rows <= 32)
+        return wide ? launch_stream_cfg<kW4A16, 2, 2, 16, 1, 4, 128>(a, cus, st)
+                    : launch_stream_cfg<kW4A16, 2, 1, 16, 1, 4, 128>(a, cus, st);
+    // (64 rows by 32 columns do not fit LDS.)
+    if (w.rows <= 48)
+        return wide ? launch_stream_cfg<kW4A16, 3, 2, 12, 2, 4, 64>(a, cus, st)
+                    : launch_stream_cfg<kW4A16, 3, 1, 12, 2, 4, 64>(a, cus, st);
+    return launch_stream_cfg<kW4A16, 4, 1, 16, 2, 4, 64>(a, cus, st);
 }
 
 // Five to 64 rows of f16 weights (up to 4 take the GEMV).

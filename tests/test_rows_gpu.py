@@ -108,7 +108,8 @@ def test_w8a16_stream(rows, width, columns):
     (1, 33024, 20), (3, 256, 5), (4, 2304, 33), (4, 4352, 2050), (3, 4352, 4100), (4, 512, 4100), (4, 256, 20000),
     (5, 256, 15), (8, 1792, 100), (7, 768, 4100), (9, 3328, 17), (16, 256, 64), (13, 1280, 4097), (17, 512, 31),
     (32, 2816, 70), (29, 768, 4129), (6, 256, 131100), (5, 128, 33), (8, 1152, 100), (16, 2944, 4099), (3, 4224, 2051),
-    (32, 1408, 65), (17, 384, 4130)])
+    (32, 1408, 65), (17, 384, 4130), (33, 128, 47), (48, 640, 4100), (40, 1408, 130), (47, 256, 131104),
+    (49, 256, 33), (64, 1152, 70), (63, 384, 4099), (56, 128, 131100)])
 def test_w4a16_stream(oracle, rows, width, columns):
     rng = np.random.default_rng(rows + 5 * width + columns)
     x = rng.standard_normal((rows, width)).astype(np.float16)
@@ -126,7 +127,8 @@ def test_w4a16_stream(oracle, rows, width, columns):
 # (2^-24 of the absolute sum for each of `width` additions), no more.
 @pytest.mark.parametrize("low,high", [(1e-6, 5e-5), (8192.0, 65536.0)])
 @pytest.mark.parametrize("rows,width,columns", [
-    (3, 256, 2100), (4, 640, 33), (8, 384, 100), (16, 512, 4200), (32, 128, 70)])
+    (3, 256, 2100), (4, 640, 33), (8, 384, 100), (16, 512, 4200), (32, 128, 70),
+    (48, 384, 40), (64, 256, 4100)])
 def test_w4a16_stream_scales(rows, width, columns, low, high):
     rng = np.random.default_rng(rows + width + columns)
     x = (rng.standard_normal((rows, width)) * (1.0 if high < 1 else 2e-3)).astype(np.float16)
