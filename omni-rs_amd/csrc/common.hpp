@@ -182,10 +182,27 @@ __device__ __forceinline__ void lds_copy16(const uint8_t* src, uint8_t* lds_dst)
 // reserved register it will not preserve: a kernel that uses this copy must
 // not also use the builtin lds_copy16 (whose m0 setup the compiler may hoist);
 // the only other m0 users on gfx950 are absent from these kernels.
+//
+// The compiler adds no wait states inside or before inline assembly, so the
+// copy brings its own: one between the write of m0 and the LDS-DMA that reads
+// it, and five between a VALU write of the base (v_readlane of an address
+// spilled to a VGPR) and a vector-memory read of it. Moving the base onto
+// itself serves for both: the scalar unit waits for a VALU's result by itself,
+// and a scalar write needs no wait before a vector-memory read. NOP waits the
+// whole time instead, which only the f16 rings are faster with (MI355X, move
+// and NOP: f16 4096 x 4096 x 12288 367 and 358 us, W8A8 4096 x 3072 x 12288
+// with its quantisation 163.3 and 165.4, W4A16 500 x 3584 x 18944 79.1 and
+// 79.7; without the waits, on another card, 357, 161.4 and 80.4).
+#define OMNI_LDS_COPY(load) "s_mov_b32 m0, %2\n\ts_mov_b64 %1, %1\n\t" load " %0, %1"
+#define OMNI_LDS_COPY_NOP(load) "s_mov_b32 m0, %2\n\ts_nop 3\n\t" load " %0, %1"
+template <bool NOP = false>
 __device__ __forceinline__ void lds_copy16_saddr(unsigned voff, const void* base, unsigned lds_byte) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds_byte)
-                 : "memory", "m0");
+    if constexpr (NOP)
+        asm volatile(OMNI_LDS_COPY_NOP("global_load_lds_dwordx4") ::"v"(voff), "s"(base), "s"(lds_byte)
+                     : "memory", "m0");
+    else
+        asm volatile(OMNI_LDS_COPY("global_load_lds_dwordx4") ::"v"(voff), "s"(base), "s"(lds_byte) : "memory", "m0");
 #endif
 }
 
@@ -193,8 +210,7 @@ __device__ __forceinline__ void lds_copy16_saddr(unsigned voff, const void* base
 // dword at lds_byte + 4 l (any 2-byte alignment of the source).
 __device__ __forceinline__ void lds_copy2_saddr(unsigned voff, const void* base, unsigned lds_byte) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_ushort %0, %1" ::"v"(voff), "s"(base), "s"(lds_byte)
-                 : "memory", "m0");
+    asm volatile(OMNI_LDS_COPY("global_load_lds_ushort") ::"v"(voff), "s"(base), "s"(lds_byte) : "memory", "m0");
 #endif
 }
 

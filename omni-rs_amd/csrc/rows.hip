@@ -74,8 +74,7 @@ struct RowsArgs {
 // 4096, the bare read: 4.05 against 4.45 us).
 __device__ __forceinline__ void lds_copy16_nt(unsigned voff, const void* base, unsigned lds_byte) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(base), "s"(lds_byte)
-                 : "memory", "m0");
+    asm volatile(OMNI_LDS_COPY("global_load_lds_dwordx4") " nt" ::"v"(voff), "s"(base), "s"(lds_byte) : "memory", "m0");
 #endif
 }
 

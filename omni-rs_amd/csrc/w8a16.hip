@@ -1524,7 +1524,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void w8a16_ring_kernel(W8A16Args a, i
         const bool is_x = c * 16 < kXR * BM;  // wave-uniform
         const uint8_t* base = is_x ? reinterpret_cast<const uint8_t*>(a.x) + kk * 64 * KP
                                    : reinterpret_cast<const uint8_t*>(a.w) + kk * kWBytes;
-        lds_copy16_saddr(voff[j], base, stage_lds[s] + c * 1024);
+        lds_copy16_saddr<WB == 16>(voff[j], base, stage_lds[s] + c * 1024);
         if constexpr (WB == 4) {
             if (j == kCpw - 1)
                 lds_copy2_saddr(voff_sc, a.gscale + (int)kk / gdiv,
