@@ -1471,6 +1471,10 @@ hipError_t launch_bn(const W8A8Args& a, hipStream_t stream) {
 // 0 or unset = the shape rule below.
 int w8a8_split_override() { return knob(Knob::W8A8Splits, 0); }
 
+// A pinned tile or split keeps the call off the streaming kernels (rows.hip),
+// which have neither.
+bool w8a8_pinned() { return w8a8_tile_override() != 0 || w8a8_split_override() > 1; }
+
 // Split K when 256 x 128 tiles fill at most half of the CUs and K >= 4608, or
 // at most an eighth of them and K >= 4096: K split up to 6 ways, at most one
 // unit per CU, on the 256 x 128 pair ring. The partial sums cost one int32
@@ -1508,7 +1512,7 @@ int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width) {
     a.columns = columns;
     a.width = width;
     if (!ring_offsets_fit(a)) return 0;
-    if (w8a8_tile_override() == 0 && rows <= 64 && w8a8_rows_fits(a)) return 0;  // no split there
+    if (!w8a8_pinned() && rows <= 64 && w8a8_rows_fits(a)) return 0;  // no split there
     const int sp = w8a8_auto_splits(rows, columns, width, num_cus());
     return sp > 1 ? (int64_t)sp * rows * columns : 0;
 }
@@ -1534,7 +1538,7 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream) {
             break;
         default: break;
     }
-    const bool pinned = w8a8_tile_override() != 0;
+    const bool pinned = w8a8_pinned();
     // Up to 64 rows the weights' stream is all that counts: on every shape
     // measured (rows.hip) the streaming kernel is ahead of 256-row tiles.
     if (!pinned && a.rows <= 64 && w8a8_rows_fits(a)) return launch_w8a8_rows(a, 0, stream);

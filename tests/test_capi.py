@@ -110,6 +110,18 @@ def test_tuning_knobs_set_unset_restore():
     assert L.omni_int8_set_tuning(None, 2, 1) == _lib.OMNI_BAD_ARGUMENT
 
 
+@pytest.mark.parametrize("rows,columns,width", [(8, 4096, 4096), (64, 1536, 8960), (256, 4096, 12288)])
+def test_a_pinned_w8a8_split_is_honoured(knobs, rows, columns, width):
+    # OMNI_W8A8_SPLITS forces split K, also where the streaming kernels
+    # (csrc/rows.hip), which have no split, would take the call.
+    knobs.set("OMNI_W8A8_SPLITS", "4")
+    assert _lib.lib().omni_w8a8_gemm_workspace_size(rows, columns, width) == 4 * rows * columns * 4
+    knobs.set("OMNI_W8A8_SPLITS", "0")  # the automatic value
+    automatic = _lib.lib().omni_w8a8_gemm_workspace_size(rows, columns, width)
+    knobs.unset("OMNI_W8A8_SPLITS")
+    assert _lib.lib().omni_w8a8_gemm_workspace_size(rows, columns, width) == automatic
+
+
 def test_no_getenv_on_launch_paths():
     # The kernels' tuning knobs are read from the environment once per
     # process (omni::knob); the only per-call reads are the reference's own

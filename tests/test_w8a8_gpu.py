@@ -587,6 +587,33 @@ def test_w8a8_split_k_bit_identical(oracle, splits, monkeypatch, knobs):
         assert torch.equal(ref_acc.double(), exact)
 
 
+@pytest.mark.parametrize("rows", [5, 64, 65, 256])
+def test_w8a8_pinned_split_runs(oracle, rows, knobs):
+    # A pinned split runs on shapes that the streaming kernels take by default,
+    # bit-identically: it writes its partial sums, they use no workspace.
+    from omni_int8 import _lib
+    L = _lib.lib()
+    width, columns = 4096, 520
+    rng = np.random.default_rng(rows)
+    codes = rng.integers(-128, 128, (rows, width), dtype=np.int8)
+    w = rng.integers(-128, 128, (columns, width), dtype=np.int8)
+    rs = rng.uniform(1e-4, 1e-2, rows).astype(np.float32)
+    scale = rng.uniform(0.002, 0.02, columns).astype(np.float32)
+    want, _ = oracle.w8a8_finish(oracle.int8_acc(codes, w), np.zeros(rows, np.int32), rs, scale,
+                                 np.zeros(columns, np.int32))
+    cd, wd, rd, sd = dev(codes), dev(w), dev(rs), dev(scale)
+    for splits in ("4", "0"):
+        knobs.set("OMNI_W8A8_SPLITS", splits)
+        ws = torch.full((4 * rows * columns * 4,), 0x5A, dtype=torch.uint8, device="cuda")
+        out = torch.empty((rows, columns), dtype=torch.float32, device="cuda")
+        st = L.omni_w8a8_gemm_ws(cd.data_ptr(), rd.data_ptr(), None, wd.data_ptr(), sd.data_ptr(), None, None, rows,
+                                 columns, width, out.data_ptr(), oi.OMNI_F32, None, oi.OMNI_LOWERING_AUTO,
+                                 ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+        assert st == 0, _lib.last_error()
+        assert np.array_equal(host(out).view(np.uint32), want.view(np.uint32)), splits
+        assert bool((ws != 0x5A).any()) == (splits == "4"), splits
+
+
 def test_w8a8_split_k_workspace_contract(monkeypatch):
     # omni_w8a8_gemm_workspace_size: the reference's 256-row benchmark shapes
     # with 32 tiles split, 256 x 12288 x 4096 (96 tiles) and the north-star
