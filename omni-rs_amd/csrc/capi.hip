@@ -111,21 +111,22 @@ std::atomic<int> g_cus[kMaxDevices];
 // unset, the measured rule below.
 int w8a16_route() { return omni::knob(omni::Knob::W8A16Route, 0); }
 
-// A knob that pins a kernel or a split keeps the call off the streaming
-// kernels (rows.hip), which have none of their own.
-bool pinned(std::initializer_list<omni::Knob> knobs) {
-    constexpr int kUnset = INT32_MIN;
-    for (omni::Knob k : knobs)
-        if (omni::knob(k, kUnset) != kUnset) return true;
-    return false;
+// A pinned kernel or split keeps the call off the streaming kernels (rows.hip),
+// which have none of their own. A knob at its automatic value pins nothing: 0,
+// for a number of splits also 1, and less than 0 for the skinny kernels' (0
+// turns theirs off).
+bool pinned(std::initializer_list<omni::Knob> kernels, omni::Knob splits, omni::Knob skinny_splits) {
+    for (omni::Knob k : kernels)
+        if (omni::knob(k, 0) != 0) return true;
+    return omni::knob(splits, 0) > 1 || omni::knob(skinny_splits, -1) >= 0;
 }
 bool w8a16_pinned() {
     using K = omni::Knob;
-    return pinned({K::W8A16Route, K::W8A16Gemv, K::W8A16Skinny, K::W8A16SkinnySplit, K::W8A16Tile, K::W8A16Splits});
+    return pinned({K::W8A16Route, K::W8A16Gemv, K::W8A16Skinny, K::W8A16Tile}, K::W8A16Splits, K::W8A16SkinnySplit);
 }
 bool w4a16_pinned() {
     using K = omni::Knob;
-    return pinned({K::W8A16Route, K::W4A16Gemv, K::W4A16SkinnySplit, K::W4A16Tile, K::W4A16Splits});
+    return pinned({K::W8A16Route, K::W4A16Gemv, K::W4A16Tile}, K::W4A16Splits, K::W4A16SkinnySplit);
 }
 
 // Where the streaming kernels do not take the call (w8a16_rows_take):

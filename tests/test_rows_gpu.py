@@ -143,6 +143,39 @@ def test_w4a16_stream_scales(rows, width, columns, low, high):
     assert fits.any() and (np.abs(got - exact) <= bound)[fits].all()
 
 
+# A knob at its automatic value leaves the choice as it is without the knob; a
+# pin keeps the call off the streaming kernels. The skinny kernel that then
+# takes this shape splits K and writes its workspace, they use none.
+@pytest.mark.parametrize("name,value,pins", [
+    ("ROUTE", 0, False), ("GEMV", 0, False), ("SKINNY", 0, False), ("TILE", 0, False), ("SPLITS", 0, False),
+    ("SPLITS", 1, False), ("SKINNY_SPLIT", -1, False), ("ROUTE", 1, True), ("SKINNY", 1, True), ("SPLITS", 2, True),
+    ("SKINNY_SPLIT", 4, True)])
+def test_automatic_knob_values_pin_nothing(name, value, pins, knobs):
+    from omni_int8 import _lib
+    L = _lib.lib()
+    rows, width, columns = 16, 4096, 14336
+    x = torch.randn((rows, width), device="cuda").half()
+    out = torch.empty((rows, columns), dtype=torch.float16, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    for int4 in (False, True):
+        if int4 and name == "SKINNY":  # W8A16's alone
+            continue
+        knobs.set(("OMNI_W4A16_" if int4 and name != "ROUTE" else "OMNI_W8A16_") + name, value)
+        ws = torch.full((4 * rows * columns * 4,), 0x5A, dtype=torch.uint8, device="cuda")
+        if int4:
+            w = torch.randint(0, 256, (columns, width // 2), dtype=torch.uint8, device="cuda")
+            scale = torch.rand((columns, width // 128), device="cuda").bfloat16()
+            st = L.omni_w4a16_gemm_ws(x.data_ptr(), w.data_ptr(), scale.data_ptr(), 128, None, rows, columns, width,
+                                      out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+        else:
+            w = torch.randint(-127, 128, (columns, width), dtype=torch.int8, device="cuda")
+            scale = torch.rand(columns, device="cuda").half()
+            st = L.omni_w8a16_gemm_ws(x.data_ptr(), w.data_ptr(), scale.data_ptr(), None, rows, columns, width,
+                                      out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+        assert st == 0, _lib.last_error()
+        assert bool((ws != 0x5A).any()) == pins, int4
+
+
 @pytest.mark.parametrize("rows,width,columns", [
     (5, 32, 9), (8, 160, 100), (9, 1056, 33), (16, 8192, 17), (17, 96, 64), (32, 544, 40), (33, 64, 31),
     (48, 1120, 70), (49, 32, 16), (64, 2080, 95)])

@@ -264,8 +264,8 @@ def test_split_k_workspace_contract(oracle, monkeypatch, knobs):
 @pytest.mark.parametrize("rows,width,columns,group", [(24, 4096, 8200, 128), (40, 2048, 16400, 64),
                                                       (40, 8192, 4100, 128), (17, 512, 300, 128)])
 def test_mid_rows_on_every_route(oracle, monkeypatch, route, rows, width, columns, group, knobs):
-    # 17..64 activation rows: the default choice (the first two shapes take
-    # the GEMM, the last two the skinny kernel), and each route forced
+    # 17..64 activation rows: the default choice (the streaming kernel, and
+    # the GEMM for the group of 64), and each route forced
     knobs.set("OMNI_W8A16_ROUTE", route)
     rng = np.random.default_rng(rows + width + columns + group)
     x, packed, bits, b = wd.random_case(rng, rows, width, columns, group, bias=True)
@@ -282,8 +282,10 @@ def test_mid_rows_on_every_route(oracle, monkeypatch, route, rows, width, column
 def test_skinny_split_k(oracle, monkeypatch, splits, rows, width, columns, group, bias, knobs):
     # The int4 split-K skinny kernel (5..16 rows): units of 64 columns x
     # K / splits, partial sums of the scaled codes added in order by the
-    # reduction (bias only); forced splits, and the default choice
-    # ("auto": K of 3072..4096 over at least 8192 columns), deterministic
+    # reduction (bias only); forced splits, and the skinny kernels' own choice
+    # ("auto": K of 3072..4096 over at least 8192 columns), deterministic. Off
+    # the streaming kernel, which takes groups of 128 by default.
+    knobs.set("OMNI_W8A16_ROUTE", "1")
     if splits != "auto":
         knobs.set("OMNI_W4A16_SKINNY_SPLIT", splits)
     rng = np.random.default_rng(rows + width + columns + group)

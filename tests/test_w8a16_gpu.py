@@ -175,13 +175,10 @@ def test_mfma_gemm_shapes(oracle, rows, width, columns):
                                                 (7, 16, 3), (40, 4096, 8200), (60, 2048, 8300),
                                                 (48, 4112, 9000)])
 def test_skinny_rows_on_both_routes(oracle, monkeypatch, route, rows, width, columns, knobs):
-    # 5..64 activation rows: the default choice (route 0), the skinny MFMA
-    # kernel (OMNI_W8A16_ROUTE=1) and the tiled MFMA GEMM (=2) against the
-    # f64 ground truth, with K tails that are not a multiple of 64 and
-    # ragged column counts; (40, 4096, 8200) and (60, 2048, 8300) take the
-    # GEMM by default, (48, 4112, 9000) stays skinny by default (no ring
-    # kernel runs K % 64 != 0, and the register-staged GEMM only pays above
-    # 48 rows).
+    # 5..64 activation rows: the default choice (route 0: mostly the
+    # streaming kernels), the skinny MFMA kernel (OMNI_W8A16_ROUTE=1) and the
+    # tiled MFMA GEMM (=2) against the f64 ground truth, with K tails that are
+    # not a multiple of 64 and ragged column counts.
     knobs.set("OMNI_W8A16_ROUTE", route)
     rng = np.random.default_rng(rows * 3 + width + columns)
     x, w, s, b = make(rng, rows, width, columns, bias=columns % 2 == 1)
@@ -198,7 +195,9 @@ def test_skinny_lds_kernel_and_fallback(oracle, monkeypatch, kernel, rows, width
     # 5..16 rows with K % 64 == 0 and K <= 4096: the LDS-staged skinny kernel
     # (0; its K = 1024 / 2048 / 3072 / 4096 builds and the run-time-K one) and
     # w8a16_skinny_kernel (OMNI_W8A16_SKINNY=1), with idle waves (K < 1024),
-    # ragged column counts and bias, against the f64 truth.
+    # ragged column counts and bias, against the f64 truth; the route is
+    # pinned, since the streaming kernels take most of these by default.
+    knobs.set("OMNI_W8A16_ROUTE", "1")
     knobs.set("OMNI_W8A16_SKINNY", kernel)
     rng = np.random.default_rng(rows * 5 + width + columns)
     x, w, s, b = make(rng, rows, width, columns, bias=True)
@@ -337,7 +336,9 @@ def test_skinny_split_k(oracle, monkeypatch, splits, rows, width, columns, bias,
     # The decode-shaped split-K kernel (5..16 rows): units of 64 columns x
     # K / splits, f32 partial sums, then the in-order reduction. Splits that
     # do not divide K into multiples of 256 of at most 1024 fall back to the
-    # unsplit kernels; ragged columns, bias, K from 256 to 12288.
+    # unsplit kernels; ragged columns, bias, K from 256 to 12288. Off the
+    # streaming kernels, which take most of these by default.
+    knobs.set("OMNI_W8A16_ROUTE", "1")
     if splits != "auto":
         knobs.set("OMNI_W8A16_SKINNY_SPLIT", splits)
     rng = np.random.default_rng(rows * 7 + width + columns + (0 if splits == "auto" else int(splits)))
