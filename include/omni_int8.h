@@ -115,11 +115,12 @@ int omni_w8a8_gemm(const int32_t* x_packed, const float* x_scale, const int32_t*
                    const float* bias, int64_t rows, int64_t columns, int64_t width, void* out,
                    int out_dtype, int32_t* acc_dump, int lowering, void* stream);
 
-/* Bytes of workspace omni_w8a8_gemm_ws uses at most for this shape on the
- * current device (a call of few rows may run without): split-K partial sums (int32 [splits][rows][columns]) for shapes
- * whose 256 x 128 output tiles alone would leave most CUs idle (the
- * reference's own 256-row benchmark shapes); 0 when the shape does not
- * split. */
+/* Bytes of workspace omni_w8a8_gemm_ws uses for this shape on the current
+ * device: split-K partial sums (int32 [splits][rows][columns]) for shapes
+ * whose 256 x 128 output tiles alone would leave most CUs idle; 0 when the
+ * shape does not split, and for few rows or small matrices (the reference's
+ * own 256-row benchmark shapes among them), which stream their weights in one
+ * launch. */
 size_t omni_w8a8_gemm_workspace_size(int64_t rows, int64_t columns, int64_t width);
 
 /* omni_w8a8_gemm with a caller-owned workspace (256-byte aligned, or NULL
@@ -237,10 +238,10 @@ int omni_w8a16_gemm(const uint16_t* x, const int8_t* w, const uint16_t* scale,
                     const uint16_t* bias, int64_t rows, int64_t columns, int64_t width,
                     uint16_t* out, void* stream);
 
-/* Bytes of workspace omni_w8a16_gemm_ws uses at most for this shape on the
- * current device (calls of up to 64 rows may run without): split-K partial sums (f32 [splits][rows][columns]) for GEMM shapes
+/* Bytes of workspace omni_w8a16_gemm_ws uses for this shape on the current
+ * device: split-K partial sums (f32 [splits][rows][columns]) for GEMM shapes
  * whose output tiles alone would leave CUs idle; 0 when the shape does not
- * split. */
+ * split, as for the up to 64 rows that stream their weights in one launch. */
 size_t omni_w8a16_gemm_workspace_size(int64_t rows, int64_t columns, int64_t width);
 
 /* omni_w8a16_gemm with a caller-owned workspace (256-byte aligned, or NULL
@@ -270,10 +271,10 @@ int omni_w4a16_gemm(const uint16_t* x, const uint8_t* w_packed, const uint16_t* 
                     int64_t group, const uint16_t* bias, int64_t rows, int64_t columns,
                     int64_t width, uint16_t* out, void* stream);
 
-/* Bytes of workspace omni_w4a16_gemm_ws uses at most for this shape on the
- * current device (calls of few rows may run without): split-K partial sums (f32 [splits][rows][columns]) for the shapes
- * that split (GEMM shapes, and 5..16 rows over long K and many columns); 0
- * when the shape does not split. No counterpart in the reference: it
+/* Bytes of workspace omni_w4a16_gemm_ws uses for this shape on the current
+ * device: split-K partial sums (f32 [splits][rows][columns]) for the shapes
+ * that split (GEMM shapes, and for groups other than 128 also 5..16 rows over
+ * long K and many columns); 0 when the shape does not split. No counterpart in the reference: it
  * serves omni_w4a16_gemm_ws. */
 size_t omni_w4a16_gemm_workspace_size(int64_t rows, int64_t columns, int64_t width, int64_t group);
 

@@ -149,8 +149,7 @@ bool midrows_take_gemm(int64_t rows, int64_t columns, int64_t width, bool int4, 
 
 // The W8A16 route apart from the streaming kernels: 0 GEMV, 1 skinny MFMA, 2
 // the GEMM. `a` gives the shape (and, for W4A16, the group and scale layout)
-// the ring check reads. The workspace sizes follow it (a call that the
-// streaming kernels take leaves its workspace unused).
+// the ring check reads.
 int w8a16_kind(const omni::W8A16Args& a) {
     const int64_t rows = a.rows, columns = a.columns, width = a.width;
     // The GEMV spreads a row over one workgroup of at most 1024 lanes, one
@@ -608,7 +607,9 @@ int omni_convrot_linear(const void* x, int x_dtype, int64_t rows, int64_t width,
 
 size_t omni_w8a16_gemm_workspace_size(int64_t rows, int64_t columns, int64_t width) {
     if (rows <= 0 || columns <= 0 || width <= 0 || width % 16 != 0) return 0;
-    switch (w8a16_kind(shape_args(rows, columns, width))) {
+    const omni::W8A16Args a = shape_args(rows, columns, width);
+    if (!w8a16_pinned() && omni::w8a16_rows_take(a)) return 0;
+    switch (w8a16_kind(a)) {
         case 1: return (size_t)omni::w8a16_skinny_partial_elems(rows, columns, width) * sizeof(float);
         case 2: return (size_t)omni::w8a16_partial_elems(rows, columns, width) * sizeof(float);
         default: return 0;
@@ -662,7 +663,9 @@ size_t omni_w4a16_gemm_workspace_size(int64_t rows, int64_t columns, int64_t wid
     if (rows <= 0 || columns <= 0 || width <= 0 || group <= 0 || width % 32 != 0 || group % 32 != 0 ||
         width % group != 0)
         return 0;
-    switch (w4a16_kind(shape_args(rows, columns, width, group))) {
+    const omni::W8A16Args a = shape_args(rows, columns, width, group);
+    if (!w4a16_pinned() && omni::w4a16_rows_take(a)) return 0;
+    switch (w4a16_kind(a)) {
         case 1: return (size_t)omni::w4a16_skinny_partial_elems(rows, columns, width) * sizeof(float);
         case 2: return (size_t)omni::w4a16_partial_elems(rows, columns, width, group) * sizeof(float);
         default: return 0;

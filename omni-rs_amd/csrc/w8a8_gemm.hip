@@ -1505,6 +1505,15 @@ hipError_t launch_w8a8_scalar(const W8A8Args& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Whether the streaming kernels' tiles (65 rows and more, estimated at us) take
+// a call that would split K: against the split's GEMM and reduction, fitted as
+// described in launch_w8a8_mfma. Whether there is room for the sums does not
+// count: then the choice is against the slower unsplit rings.
+static bool tiles_beat_split(const W8A8Args& a, double us) {
+    const double m = (double)a.rows / 256.0, mb = 1e-6 * (double)a.width * (double)a.columns;
+    return us < 13.0 + 0.22 * mb + m * (5.0 + 0.09 * mb);
+}
+
 int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width) {
     if (rows <= 0 || columns <= 0 || width % 64 != 0) return 0;
     W8A8Args a{};
@@ -1512,8 +1521,11 @@ int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width) {
     a.columns = columns;
     a.width = width;
     if (!ring_offsets_fit(a)) return 0;
-    if (!w8a8_pinned() && rows <= 64 && w8a8_rows_fits(a)) return 0;  // no split there
     const int sp = w8a8_auto_splits(rows, columns, width, num_cus());
+    if (sp > 1 && !w8a8_pinned() && w8a8_rows_fits(a)) {  // the streaming kernels need none
+        int nb;
+        if (rows <= 64 || tiles_beat_split(a, w8a8_rows_us(rows, columns, width, &nb))) return 0;
+    }
     return sp > 1 ? (int64_t)sp * rows * columns : 0;
 }
 
@@ -1586,13 +1598,9 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream) {
     const int64_t kt = a.width / 64;
     const int sp = w8a8_auto_splits(a.rows, a.columns, a.width, cus);
     if (sp > 1) {
+        if (tiles_beat_split(a, 0.95 * tiles_us)) return launch_w8a8_rows(a, tiles_nb, stream);
         const int64_t tiles = ((a.rows + 255) / 256) * ((a.columns + 127) / 128);
-        if (fit_splits(a, tiles, (int)kt, sp) > 1) {
-            // The GEMM and its reduction, us.
-            const double m = (double)a.rows / 256.0, mb = 1e-6 * K * (double)a.columns;
-            if (0.95 * tiles_us < 13.0 + 0.22 * mb + m * (5.0 + 0.09 * mb)) return launch_w8a8_rows(a, tiles_nb, stream);
-            return launch_pair<128>(a, stream, sp);
-        }
+        if (fit_splits(a, tiles, (int)kt, sp) > 1) return launch_pair<128>(a, stream, sp);
     }
     Cand best{cost(243.7, 117070.0, 256, 192), 16};
     auto consider = [&](bool ok, double t, int id) {

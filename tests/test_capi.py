@@ -122,6 +122,27 @@ def test_a_pinned_w8a8_split_is_honoured(knobs, rows, columns, width):
     assert _lib.lib().omni_w8a8_gemm_workspace_size(rows, columns, width) == automatic
 
 
+def test_streamed_calls_ask_for_no_workspace(knobs):
+    # The weight-streaming kernels (csrc/rows.hip) need none, so the size
+    # queries ask for none where they take the call; a pin that keeps the call
+    # off them brings the split's size back. Shapes that split K before.
+    L = _lib.lib()
+    for rows, columns, width in ((16, 14336, 4096), (24, 14336, 4096), (32, 18944, 3584)):
+        assert L.omni_w8a16_gemm_workspace_size(rows, columns, width) == 0, (rows, columns, width)
+        assert L.omni_w4a16_gemm_workspace_size(rows, columns, width, 128) == 0, (rows, columns, width)
+    for rows, columns, width in ((32, 4096, 4096), (256, 4096, 4096), (128, 4096, 8192), (256, 4096, 12288)):
+        assert L.omni_w8a8_gemm_workspace_size(rows, columns, width) == 0, (rows, columns, width)
+    # these still split
+    assert L.omni_w8a8_gemm_workspace_size(512, 4096, 12288) >= 2 * 512 * 4096 * 4
+    assert L.omni_w8a16_gemm_workspace_size(256, 4096, 4096) >= 2 * 256 * 4096 * 4
+    assert L.omni_w4a16_gemm_workspace_size(16, 14336, 4096, 64) == 4 * 16 * 14336 * 4
+    knobs.set("OMNI_W8A16_ROUTE", "1")
+    assert L.omni_w8a16_gemm_workspace_size(16, 14336, 4096) == 4 * 16 * 14336 * 4
+    assert L.omni_w4a16_gemm_workspace_size(16, 14336, 4096, 128) == 4 * 16 * 14336 * 4
+    knobs.set("OMNI_W8A8_TILE", "17")  # the ring that splits
+    assert L.omni_w8a8_gemm_workspace_size(256, 4096, 4096) >= 2 * 256 * 4096 * 4
+
+
 def test_no_getenv_on_launch_paths():
     # The kernels' tuning knobs are read from the environment once per
     # process (omni::knob); the only per-call reads are the reference's own

@@ -300,9 +300,10 @@ def test_skinny_split_k(oracle, monkeypatch, splits, rows, width, columns, group
     assert torch.equal(got, again)
 
 
-def test_skinny_split_k_workspace_size():
+def test_skinny_split_k_workspace_size(knobs):
     from omni_int8 import _lib
     L = _lib.lib()
+    knobs.set("OMNI_W8A16_ROUTE", "1")  # off the streaming kernel, which needs no workspace
     assert L.omni_w4a16_gemm_workspace_size(16, 14336, 4096, 128) == 4 * 16 * 14336 * 4
     assert L.omni_w4a16_gemm_workspace_size(8, 8192, 3072, 128) == 3 * 8 * 8192 * 4
     assert L.omni_w4a16_gemm_workspace_size(16, 4096, 4096, 128) == 0     # one round of workgroups

@@ -354,9 +354,10 @@ def test_skinny_split_k(oracle, monkeypatch, splits, rows, width, columns, bias,
     assert tolerance.rel_err(host(plain), ref) <= tolerance.FP16_REL_TOL
 
 
-def test_skinny_split_k_workspace_size():
+def test_skinny_split_k_workspace_size(knobs):
     from omni_int8 import _lib
     L = _lib.lib()
+    knobs.set("OMNI_W8A16_ROUTE", "1")  # off the streaming kernels, which need no workspace
     # split where the unsplit kernel needs more than one round of 16-column
     # workgroups (N > 16 x 256 CUs), K <= 4096
     assert L.omni_w8a16_gemm_workspace_size(16, 14336, 4096) == 4 * 16 * 14336 * 4
@@ -367,7 +368,8 @@ def test_skinny_split_k_workspace_size():
     assert L.omni_w8a16_gemm_workspace_size(16, 18944, 3584) == 4 * 16 * 18944 * 4  # 896-element units
     assert L.omni_w8a16_gemm_workspace_size(16, 8192, 8192) == 0                   # K > 4096
     assert L.omni_w8a16_gemm_workspace_size(17, 4096, 4096) == 0                   # skinny, not split
-    # 17 rows of a 58.7 M-weight matrix take the GEMM, split K (64 x 128 tiles)
+    # 17 rows of a 58.7 M-weight matrix in the GEMM, split K
+    knobs.set("OMNI_W8A16_ROUTE", "2")
     assert L.omni_w8a16_gemm_workspace_size(17, 14336, 4096) % (17 * 14336 * 4) == 0
     assert L.omni_w8a16_gemm_workspace_size(17, 14336, 4096) >= 2 * 17 * 14336 * 4
 

@@ -430,13 +430,13 @@ def test_north_star_try_int8_gemm_as_benched(oracle, width, columns):
 
 
 @pytest.mark.parametrize("columns,width", [(4096, 4096), (12288, 4096), (4096, 12288)])
-def test_try_int8_gemm_split_k_reference_shapes(oracle, columns, width):
+def test_try_int8_gemm_split_k_reference_shapes(oracle, columns, width, knobs):
     # The reference's own 256-row int8 GEMM benchmark shapes
     # (docs/qwen-image-convrot-optimization-research.md:5) through the
     # operator. With omni_try_int8_gemm_split_workspace_size bytes the GEMM
-    # splits K where that pays (256 x 4096 from K = 4096 on; 256 x 12288 has
-    # 96 tiles and does not split), with a workspace handed over full of
-    # garbage: every output bit equal to the unsplit operator's (the plain
+    # splits K (256 x 4096, pinned to six ways: by default these stream their
+    # weights; 256 x 12288 does not split), with a workspace handed over full
+    # of garbage: every output bit equal to the unsplit operator's (the plain
     # workspace), to a second call on the same workspace, to the no-alloc
     # entry (whose static scratch holds the split too), and to the C oracle
     # on sampled rows, with zero points.
@@ -449,6 +449,8 @@ def test_try_int8_gemm_split_k_reference_shapes(oracle, columns, width):
     scale = rng.uniform(0.002, 0.02, columns).astype(np.float32)
     zero = rng.integers(-3, 4, columns).astype(np.int32)
     xd, wp, sd, zd = dev(x), dev(w).view(torch.int32).reshape(-1), dev(scale), dev(zero)
+    if columns == 4096:
+        knobs.set("OMNI_W8A8_SPLITS", "6")
     plain_bytes = L.omni_try_int8_gemm_workspace_size(rows, width)
     split_bytes = L.omni_try_int8_gemm_split_workspace_size(rows, columns, width)
     assert (split_bytes > plain_bytes) == (columns == 4096), (plain_bytes, split_bytes)
@@ -614,17 +616,18 @@ def test_w8a8_pinned_split_runs(oracle, rows, knobs):
         assert bool((ws != 0x5A).any()) == (splits == "4"), splits
 
 
-def test_w8a8_split_k_workspace_contract(monkeypatch):
-    # omni_w8a8_gemm_workspace_size: the reference's 256-row benchmark shapes
-    # with 32 tiles split, 256 x 12288 x 4096 (96 tiles) and the north-star
-    # shapes do not; omni_w8a8_gemm_ws splits less with a smaller workspace
-    # and not at all with none, bit-identically.
+def test_w8a8_split_k_workspace_contract(knobs):
+    # omni_w8a8_gemm_workspace_size: shapes of 32 to 64 tiles over K = 12288
+    # split; smaller ones, which stream their weights, 256 x 12288 x 4096 (96
+    # tiles) and 4096-row shapes do not; omni_w8a8_gemm_ws splits less with a
+    # smaller workspace and not at all with none, bit-identically.
     from omni_int8 import _lib
     L = _lib.lib()
-    for m, n, k in ((256, 4096, 12288), (256, 4096, 4096)):
+    for m, n, k in ((512, 4096, 12288), (256, 8192, 12288)):
         size = L.omni_w8a8_gemm_workspace_size(m, n, k)
         assert size >= 2 * m * n * 4 and size % (m * n * 4) == 0, (m, n, k, size)
-    for m, n, k in ((256, 12288, 4096), (512, 4096, 4096), (4096, 12288, 3072), (4096, 3072, 12288)):
+    for m, n, k in ((256, 4096, 4096), (256, 4096, 12288), (256, 12288, 4096), (512, 4096, 4096),
+                    (4096, 12288, 3072), (4096, 3072, 12288)):
         assert L.omni_w8a8_gemm_workspace_size(m, n, k) == 0, (m, n, k)
     rows, width, columns = 256, 8192, 1024
     rng = np.random.default_rng(91)
@@ -635,6 +638,7 @@ def test_w8a8_split_k_workspace_contract(monkeypatch):
     total = dev(rng.integers(-5000, 5000, rows).astype(np.int32))
     zero = dev(rng.integers(-3, 4, columns).astype(np.int32))
     ref = oi.w8a8_gemm(codes, rs, total, w, scale, zero)
+    knobs.set("OMNI_W8A8_SPLITS", "4")
     stream = torch.cuda.current_stream().cuda_stream
     for nbytes in (4 * rows * columns * 4, (2 * rows * columns + 3) * 4, 0):
         ws = torch.full((max(nbytes, 1),), 0x5A, dtype=torch.uint8, device="cuda")
