@@ -1,8 +1,8 @@
 // Linears of a few rows on gfx950 (W8A8, and int8, int4 or f16 weights under
 // f16 activations), bound by the stream of their weights; the matrix cores
-// need a fraction of its time. Up to 64 rows one workgroup sees them all;
-// more (small matrices, where 256-row tiles would leave most CUs idle) are cut
-// into tiles of 48 or 64.
+// need a fraction of its time. Up to 64 rows one workgroup sees them all; more
+// (W8A8 on small matrices, where 256-row tiles would leave most CUs idle) are
+// cut into tiles of 48 or 64.
 //
 // A workgroup of KW waves walks blocks of 16 NB columns (units), each wave a
 // KW-th of K, in tiles of TB bytes of K. Everything a tile needs, 16 NB
@@ -488,12 +488,11 @@ int64_t row_units(int64_t rows, int64_t columns, int nb) {
 
 // More than 64 rows: tiles of 48 or 64 rows by 16 NB columns, K split over
 // four waves that each own a ring.
-template <int WK, int NB, int TB>
+template <int NB>
 hipError_t launch_tiles(const RowsArgs& a, hipStream_t st) {
     const int64_t cus = num_cus();
-    constexpr int kXC = 16 * TB * x_bytes(WK) / 1024;  // copies per 16 rows
-    return row_blocks(a.rows) == 3 ? launch_stream_cfg<WK, 3, NB, 3 * kXC, 2, 4, TB, true>(a, cus, st)
-                                   : launch_stream_cfg<WK, 4, NB, 4 * kXC, 2, 4, TB, true>(a, cus, st);
+    return row_blocks(a.rows) == 3 ? launch_stream_cfg<kW8A8, 3, NB, 6, 2, 4, 128, true>(a, cus, st)
+                                   : launch_stream_cfg<kW8A8, 4, NB, 8, 2, 4, 128, true>(a, cus, st);
 }
 
 RowsArgs f16_args(const W8A16Args& w, int64_t row_bytes) {
@@ -536,7 +535,7 @@ hipError_t launch_w8a8_rows(const W8A8Args& w, int nb, hipStream_t st) {
     a.acc_dump = w.acc_dump;
     a.out_f16 = w.out_f16;
     if (a.rows <= 64) return launch_even<kW8A8>(a, st);
-    return nb == 2 ? launch_tiles<kW8A8, 2, 128>(a, st) : launch_tiles<kW8A8, 4, 128>(a, st);
+    return nb == 2 ? launch_tiles<2>(a, st) : launch_tiles<4>(a, st);
 }
 
 // Time in us of 65 rows and more in blocks of 32 or 64 columns, fitted to 65
@@ -593,11 +592,6 @@ hipError_t launch_w8a16_rows(const W8A16Args& w, hipStream_t st) {
     const RowsArgs a = f16_args(w, w.width);
     const int64_t cus = num_cus();
     const bool wide = is_wide(a.columns, cus);
-    // Blocks of 32 columns while one round holds them (128 rows of 4096 x 4096
-    // 14.9 against 19.0 us), else of 64.
-    if (w.rows > 64)
-        return row_units(a.rows, a.columns, 2) <= cus ? launch_tiles<kW8A16, 2, 64>(a, st)
-                                                      : launch_tiles<kW8A16, 4, 64>(a, st);
     // Wide: two four-wave workgroups per CU, or from K = 4096 and 9 rows on
     // blocks of 32 columns (8 rows of 4096 x 6144 7.7 against 8.8 us, of 1536
     // x 17920 9.7 against 8.7; 16 rows of 4096 x 14336 16.5 against 21.4).

@@ -86,9 +86,20 @@ def close(got, want):
     (1, 18944, 40), (4, 16400, 33), (3, 4112, 17), (4, 1552, 8195), (5, 16, 7), (6, 1040, 100), (8, 4624, 4100),
     (8, 1168, 4112), (9, 4112, 64), (16, 240, 31), (13, 4096, 4113), (16, 528, 9000), (17, 64, 16), (32, 1104, 50),
     (31, 336, 4130), (33, 272, 40), (48, 1040, 300), (47, 368, 4100), (49, 144, 30), (64, 2064, 70), (63, 400, 4101),
-    (24, 32, 131200), (65, 1536, 33), (96, 80, 64), (97, 4608, 65), (128, 208, 130), (192, 4304, 100), (256, 64, 515),
-    (300, 48, 2100), (130, 1168, 4300), (2049, 16, 900)])
+    (24, 32, 131200)])
 def test_w8a16_stream(rows, width, columns):
+    w8a16_case(rows, width, columns)
+
+
+# More rows, which the GEMMs take: small matrices, ragged and K % 64 != 0.
+@pytest.mark.parametrize("rows,width,columns", [
+    (65, 1536, 33), (96, 80, 64), (97, 4608, 65), (128, 208, 130), (192, 4304, 100), (256, 64, 515), (300, 48, 2100),
+    (130, 1168, 4300), (2049, 16, 900)])
+def test_w8a16_above_64_rows(rows, width, columns):
+    w8a16_case(rows, width, columns)
+
+
+def w8a16_case(rows, width, columns):
     rng = np.random.default_rng(rows + 3 * width + columns)
     x = rng.standard_normal((rows, width)).astype(np.float16)
     w = rng.integers(-128, 128, (columns, width), dtype=np.int8)
