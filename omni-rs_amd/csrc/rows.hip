@@ -456,9 +456,10 @@ template <int WK>
 hipError_t launch_even(const RowsArgs& a, hipStream_t st) {
     const int64_t cus = num_cus();
     const bool wide = is_wide(a.columns, cus);
-    if (a.rows <= 4)
-        return wide ? launch_stream_cfg<WK, 1, 1, 1, 2, 4, 256>(a, cus, st)
-                    : launch_stream_cfg<WK, 1, 1, 1, 3, 8, 256>(a, cus, st);
+    if constexpr (WK == kW8A8)  // (up to 4 rows of f16 weights take the GEMV)
+        if (a.rows <= 4)
+            return wide ? launch_stream_cfg<WK, 1, 1, 1, 2, 4, 256>(a, cus, st)
+                        : launch_stream_cfg<WK, 1, 1, 1, 3, 8, 256>(a, cus, st);
     if (a.rows <= 8)
         return wide ? launch_stream_cfg<WK, 1, 1, 2, 2, 4, 256>(a, cus, st)
                     : launch_stream_cfg<WK, 1, 1, 2, 2, 8, 256>(a, cus, st);

@@ -513,7 +513,8 @@ typedef float v4f_t __attribute__((ext_vector_type(4)));
 // B use the same lane-to-k map, so each product pairs matching k and the 64
 // k of the step are summed exactly once. The 16 waves' 16 x 16 partial tiles
 // are reduced through LDS; scale (and bias) are applied once per output.
-// WB = 16: f16 weights (32 bytes per lane per step), no scale.
+// WB = 16: f16 weights (32 bytes per lane per step), no scale; only rows past
+// the GEMV's (up to 4) or the streaming kernel's (rows.hip) longest K come here.
 template <int MB, int WB = 8>
 __global__ __launch_bounds__(1024) void w8a16_skinny_kernel(W8A16Args a) {
     __shared__ float s_part[16][MB][256];
@@ -628,7 +629,7 @@ __global__ __launch_bounds__(1024) void w8a16_skinny_kernel(W8A16Args a) {
 // same kernel with K read at run time).
 constexpr int kSkinnyLdsMaxK = 4096;
 
-template <int WB, int KF = 0>
+template <int KF = 0>
 __global__ __launch_bounds__(1024) void w8a16_skinny_lds_kernel(W8A16Args a) {
     static_assert(KF % 1024 == 0 && KF <= kSkinnyLdsMaxK, "KF: a multiple of 1024 up to the maximum");
     constexpr int kK = KF > 0 ? KF : kSkinnyLdsMaxK;   // K the LDS and the unrolled loops are sized for
@@ -666,16 +667,14 @@ __global__ __launch_bounds__(1024) void w8a16_skinny_lds_kernel(W8A16Args a) {
             xv[i] = reinterpret_cast<const uint4*>(a.x + rowv[i] * K)[colv[i]];
     }
     const int64_t wn = n0 + r16 < a.columns ? n0 + r16 : a.columns - 1;  // clamped: never stored
-    const uint8_t* wrow = reinterpret_cast<const uint8_t*>(a.w) + wn * K * (WB / 8);
+    const uint8_t* wrow = reinterpret_cast<const uint8_t*>(a.w) + wn * K;
     typedef unsigned v4u __attribute__((ext_vector_type(4)));
-    v4u wv[kMaxSteps][WB / 8];
+    v4u wv[kMaxSteps];
 #pragma unroll
     for (int j = 0; j < kMaxSteps; ++j) {
         const int st = wave + 16 * j;
         const int64_t k = (int64_t)(KF > 0 || st < steps ? st : steps - 1) * 64 + 16 * g;
-#pragma unroll
-        for (int u = 0; u < WB / 8; ++u)
-            wv[j][u] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(wrow + k * (WB / 8)) + u);
+        wv[j] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(wrow + k));
     }
 #pragma unroll
     for (int i = 0; i < kMaxPieces; ++i)
@@ -686,19 +685,13 @@ __global__ __launch_bounds__(1024) void w8a16_skinny_lds_kernel(W8A16Args a) {
     for (int j = 0; j < kMaxSteps; ++j) {
         const int st = wave + 16 * j;
         if (KF == 0 && st >= steps) break;  // wave-uniform
-        v8h b0, b1;
-        if constexpr (WB == 8) {
-            v2h h[8];
-            i8x4_to_f16x4(wv[j][0].x, h[0], h[1]);
-            i8x4_to_f16x4(wv[j][0].y, h[2], h[3]);
-            i8x4_to_f16x4(wv[j][0].z, h[4], h[5]);
-            i8x4_to_f16x4(wv[j][0].w, h[6], h[7]);
-            b0 = v8h{h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
-            b1 = v8h{h[4][0], h[4][1], h[5][0], h[5][1], h[6][0], h[6][1], h[7][0], h[7][1]};
-        } else {
-            __builtin_memcpy(&b0, &wv[j][0], 16);
-            __builtin_memcpy(&b1, &wv[j][WB / 8 - 1], 16);
-        }
+        v2h h[8];
+        i8x4_to_f16x4(wv[j].x, h[0], h[1]);
+        i8x4_to_f16x4(wv[j].y, h[2], h[3]);
+        i8x4_to_f16x4(wv[j].z, h[4], h[5]);
+        i8x4_to_f16x4(wv[j].w, h[6], h[7]);
+        const v8h b0 = v8h{h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
+        const v8h b1 = v8h{h[4][0], h[4][1], h[5][0], h[5][1], h[6][0], h[6][1], h[7][0], h[7][1]};
         const uint8_t* px = sx + r16 * RS + (64 * st + 16 * g) * 2;
         v8h a0, a1;
         __builtin_memcpy(&a0, px, 16);
@@ -719,8 +712,7 @@ __global__ __launch_bounds__(1024) void w8a16_skinny_lds_kernel(W8A16Args a) {
 #pragma unroll
             for (int w = 0; w < 16; ++w) sum += s_part[w * 256 + tid];
             const float bi = a.bias ? (float)a.bias[n] : 0.0f;
-            const float sc = WB == 8 ? (float)a.scale[n] : 1.0f;
-            a.out[m * a.columns + n] = (_Float16)(sum * sc + bi);
+            a.out[m * a.columns + n] = (_Float16)(sum * (float)a.scale[n] + bi);
         }
     }
 }
@@ -889,17 +881,17 @@ hipError_t launch_skinny(const W8A16Args& a, hipStream_t stream) {
     if constexpr (WB == 8) {
         const int sp = skinny_splits(a.rows, a.width, a.columns, a.partial ? a.partial_elems : 0, cu_count());
         if (sp > 1) return launch_skinny_split(a, sp, stream);
-    }
-    if (a.rows <= 16 && a.width % 64 == 0 && a.width <= kSkinnyLdsMaxK && skinny_route() != 1) {
-        const dim3 grid((unsigned)((a.columns + 15) / 16)), block(1024);
-        switch (a.width) {
-            case 1024: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<WB, 1024>), grid, block, 0, stream, a); break;
-            case 2048: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<WB, 2048>), grid, block, 0, stream, a); break;
-            case 3072: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<WB, 3072>), grid, block, 0, stream, a); break;
-            case 4096: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<WB, 4096>), grid, block, 0, stream, a); break;
-            default: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<WB>), grid, block, 0, stream, a);
+        if (a.rows <= 16 && a.width % 64 == 0 && a.width <= kSkinnyLdsMaxK && skinny_route() != 1) {
+            const dim3 grid((unsigned)((a.columns + 15) / 16)), block(1024);
+            switch (a.width) {
+                case 1024: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<1024>), grid, block, 0, stream, a); break;
+                case 2048: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<2048>), grid, block, 0, stream, a); break;
+                case 3072: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<3072>), grid, block, 0, stream, a); break;
+                case 4096: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<4096>), grid, block, 0, stream, a); break;
+                default: hipLaunchKernelGGL((w8a16_skinny_lds_kernel<>), grid, block, 0, stream, a);
+            }
+            return hipGetLastError();
         }
-        return hipGetLastError();
     }
     if (a.rows <= 16) return launch_skinny_cfg<1, WB>(a, stream);
     if (a.rows <= 32) return launch_skinny_cfg<2, WB>(a, stream);

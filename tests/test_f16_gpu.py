@@ -106,7 +106,20 @@ def test_gemv_every_configuration(oracle, monkeypatch, cfg, knobs):
                                       (8, 1024, 256), (16, 4096, 1000), (12, 2048, 64),
                                       (6, 3072, 130)])
 def test_skinny_rows(oracle, rows, k, n):
-    # 5..64 rows (and rows past the GEMV's widest row) run the skinny MFMA kernel.
+    # 5..64 rows run the streaming kernel, fewer past the GEMV's widest row the
+    # skinny one.
+    skinny_case(oracle, rows, k, n)
+
+
+@pytest.mark.parametrize("rows,k,n", [(2, 131104, 20), (16, 131104, 16), (17, 131136, 7), (40, 131104, 18),
+                                      (64, 131104, 17)])
+def test_rows_past_the_streaming_kernel(oracle, rows, k, n):
+    # K past the streaming kernel's limit of 131072: the skinny MFMA kernel, a
+    # build per 16 rows.
+    skinny_case(oracle, rows, k, n)
+
+
+def skinny_case(oracle, rows, k, n):
     rng = np.random.default_rng(rows * 7 + k + n)
     x = torch.from_numpy(rng.standard_normal((rows, k)).astype(np.float16)).cuda()
     w = torch.from_numpy((rng.standard_normal((n, k)) * 0.02).astype(np.float16)).cuda()
