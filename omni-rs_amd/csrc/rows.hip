@@ -562,7 +562,12 @@ double w8a8_rows_us(int64_t rows, int64_t columns, int64_t width, int* nb) {
 // 21.4 (18944 x 3584). The others keep:
 //  * up to 16 rows at K = 1024, 2048, 3072, 4096 in one round of workgroups,
 //    the LDS skinny kernel built for that K (16 of 4096 x 4096 6.9 against
-//    7.5 us, of 1024 x 4096 3.4 against 3.8);
+//    7.5 us, of 1024 x 4096 3.4 against 3.8), and past it while its second
+//    round costs less than a few rows' wide blocks (5 of 1024 x 4112 3.2
+//    against 3.6, of 1024 x 8192 4.0 against 4.3, 8 even; 12 of 1024 x 4112
+//    3.5 against 3.9, from 4352 on even; 5 of 2048 x 4112 4.65 against 4.9,
+//    of 2048 x 7168 5.45 against 5.55, 8 even; 5 of 3072 x 4112 7.3 against
+//    5.9);
 //  * three and four rows, the GEMV up to K = 4096 on up to 8192 columns (4 of
 //    4096 x 4096 5.8 against 6.1, 3 of 5120 x 5120 9.0 against 9.4) and at K =
 //    4096 up to 64 M weights (4 of 4096 x 14336 13.9 against 14.5; beyond, 4
@@ -574,7 +579,8 @@ double w8a8_rows_us(int64_t rows, int64_t columns, int64_t width, int* nb) {
 //    against 17.5, of 8960 x 1536 24.4 against 37.1).
 bool w8a16_rows_take(const W8A16Args& a) {
     if (a.rows > 64 || a.width % 16 != 0 || a.width < 16 || a.width > kMaxRowBytes) return false;
-    const bool wide = is_wide(a.columns, num_cus());
+    const int64_t cus = num_cus();
+    const bool wide = is_wide(a.columns, cus);
     const double elems = (double)a.columns * (double)a.width;
     if (a.width > 16384 && a.rows <= 4) return true;
     if (a.rows <= 2) return false;
@@ -582,7 +588,11 @@ bool w8a16_rows_take(const W8A16Args& a) {
         if (a.width == 4096 && elems <= (64 << 20)) return false;
         return wide ? a.columns >= 8192 : a.width > 4096;
     }
-    if (a.rows <= 16) return wide || a.width > 4096 || a.width % 1024 != 0;
+    if (a.rows <= 16) {
+        if (a.width > 4096 || a.width % 1024 != 0) return true;
+        if (a.width == 1024) return a.columns > (a.rows <= 8 ? 32 : 17) * cus;
+        return a.width == 2048 && a.rows < 8 ? a.columns >= 32 * cus : wide;
+    }
     if (a.rows <= 32) return true;
     if (a.rows <= 48) return !wide || elems <= 36e6;
     return elems < 16e6 || (a.width <= 4096 && elems <= 26e6);

@@ -154,6 +154,25 @@ def test_w4a16_stream_scales(rows, width, columns, low, high):
     assert fits.any() and (np.abs(got - exact) <= bound)[fits].all()
 
 
+# Just past one round of its workgroups the LDS skinny kernel (route 1) keeps a
+# few rows of short K; elsewhere the streaming kernel's sums, in another order,
+# differ in some output's last bit.
+@pytest.mark.parametrize("rows,width,columns,skinny", [
+    (5, 1024, 4096, True), (5, 1024, 4112, True), (8, 1024, 8192, True), (8, 1024, 8208, False),
+    (16, 1024, 4352, True), (16, 1024, 4368, False), (7, 2048, 8176, True), (7, 2048, 8192, False),
+    (8, 2048, 4112, False), (5, 3072, 4112, False), (5, 1040, 4096, False)])
+def test_w8a16_short_k_past_one_round(rows, width, columns, skinny, knobs):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the columns are those of 256 CUs")
+    g = torch.Generator(device="cuda").manual_seed(rows + width + columns)
+    x = torch.randn((rows, width), generator=g, device="cuda").half()
+    w = torch.randint(-127, 128, (columns, width), generator=g, device="cuda", dtype=torch.int8)
+    scale = torch.rand(columns, generator=g, device="cuda").half()
+    got = oi.w8a16_linear(x, w, scale)
+    knobs.set("OMNI_W8A16_ROUTE", "1")
+    assert torch.equal(got, oi.w8a16_linear(x, w, scale)) == skinny
+
+
 # A knob at its automatic value leaves the choice as it is without the knob; a
 # pin keeps the call off the streaming kernels. The skinny kernel that then
 # takes this shape splits K and writes its workspace, they use none.
