@@ -63,8 +63,8 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream);
 // current device (0: no split); with fewer in W8A8Args it splits less.
 int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width);
 hipError_t launch_w8a8_scalar(const W8A8Args& a, hipStream_t stream);
-// The weight-streaming kernels for few rows (rows.hip); no workspace. Above 64
-// rows: their estimated time in us, and the column blocks (2 or 4) it is for.
+// The weight-streaming kernels for few rows (rows.hip); no workspace. Their
+// estimated time in us, and above 64 rows the column blocks (2 or 4) it is for.
 bool w8a8_rows_fits(const W8A8Args& a);
 double w8a8_rows_us(int64_t rows, int64_t columns, int64_t width, int* nb);
 hipError_t launch_w8a8_rows(const W8A8Args& a, int nb, hipStream_t stream);

@@ -542,15 +542,35 @@ hipError_t launch_w8a8_rows(const W8A8Args& w, int nb, hipStream_t st) {
 // Time in us of 65 rows and more in blocks of 32 or 64 columns, fitted to 65
 // to 1024 rows of thirteen K x N (1152 ... 14336 x 1152 ... 28672): each round
 // of one tile per CU costs a fixed part and its K loop (within 10 % of 64 of
-// the 78 timings, 20 % of the rest).
+// the 78 timings, 20 % of the rest). Of 17 to 64 rows, for K from 6000 on: up
+// to one block of 16 columns per CU the K loop of a block and its share of the
+// weights' stream; wider, rounds of one block of 32 per CU, a partial last one
+// from half a round up (1100 timings: within 4 % of half, 10 % of nine in
+// ten). Rows of the weights that are not whole 128-byte lines take 1.3 times
+// as long, above 64 rows 1.2 (1300 timings). Fewer rows are ahead of every other kernel (1).
 double w8a8_rows_us(int64_t rows, int64_t columns, int64_t width, int* nb) {
     const int64_t cus = num_cus();
+    *nb = 0;
+    if (rows <= 16) return 1.0;
+    const double K = 1e-3 * (double)width;
+    const double line = width % 128 == 0 ? 1.0 : rows <= 64 ? 1.3 : 1.2;
+    if (rows <= 64) {
+        const int mb = (int)((rows + 15) / 16) - 2;
+        if (!is_wide(columns, cus)) {
+            constexpr double kLoop[3] = {0.58, 0.89, 1.06};
+            return 3.8 + K * (kLoop[mb] * line + 1.05e-3 * (double)((columns + 15) / 16));
+        }
+        constexpr double kFull[3] = {1.55, 1.80, 2.16}, kPart[3] = {1.0, 1.12, 1.22};
+        const int64_t units = (columns + 31) / 32, rem = units % cus;
+        const double part = rem ? kPart[mb] + 0.65 * (double)rem / (double)cus : 0.0;
+        return 3.3 + line * K * ((double)(units / cus) * kFull[mb] + part);
+    }
     const int mb = row_blocks(rows);
     auto us = [&](int n, double fixed, double per_k) {
         const int64_t rounds = (row_units(rows, columns, n) + cus - 1) / cus;
-        return 5.0 + (double)rounds * (fixed + per_k * (double)width * (mb + n) / (4 + n));
+        return 5.0 + (double)rounds * (fixed + per_k * line * K * (mb + n) / (4 + n));
     };
-    const double t2 = us(2, 1.3, 0.0015), t4 = us(4, 2.1, 0.00206);
+    const double t2 = us(2, 1.3, 1.5), t4 = us(4, 2.1, 2.06);
     *nb = t2 < t4 ? 2 : 4;
     return t2 < t4 ? t2 : t4;
 }

@@ -1505,14 +1505,107 @@ hipError_t launch_w8a8_scalar(const W8A8Args& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Whether the streaming kernels' tiles (65 rows and more, estimated at us) take
-// a call that would split K: against the split's GEMM and reduction, fitted as
-// described in launch_w8a8_mfma. Whether there is room for the sums does not
-// count: then the choice is against the slower unsplit rings.
-static bool tiles_beat_split(const W8A8Args& a, double us) {
-    const double m = (double)a.rows / 256.0, mb = 1e-6 * (double)a.width * (double)a.columns;
-    return us < 13.0 + 0.22 * mb + m * (5.0 + 0.09 * mb);
+namespace {
+
+// What runs a W8A8 call: the streaming kernels (id: their column blocks), split
+// K on the 256 x 128 pair ring (splits > 1), or a kernel as OMNI_W8A8_TILE
+// numbers them, unsplit.
+struct W8A8Plan {
+    bool stream;
+    int id, splits;
+};
+
+// Cost model, fitted to MI355X timings of every candidate on ten shapes
+// (prefill GEMMs of 2048 and 4096 rows and the reference's 256-row benchmark
+// shapes; codes of N(0,1) rows and uniform weights rotated past the MALL, f32
+// out): a kernel runs its tiles in rounds of one tile per CU, a round costs
+// BM * BN * (c * K + e) (c: per output element and K byte; e: the per-tile
+// prologue and epilogue), and a partial last round with fill f costs
+// (0.7 + 0.3 f) of a full one (the chip is power-limited on this path, so a
+// partly idle round runs at a higher clock). It picks the fastest candidate,
+// or one within 1 %, on all ten operands rotated; the other kernels
+// (register-staged, two-waves-per-SIMD DMA, single-refill rings at 256 x 192
+// and 256 x 128) lost on every one and stay reachable through OMNI_W8A8_TILE.
+//
+// Where the tiles leave CUs idle, the others compete by fitted times in us:
+//  * whole: the cost model's (in fs) plus 2.5, 1.2 times it for the
+//    register-staged kernels;
+//  * split K (split_us): 1200 timings of 5 to 2000 rows, K 8192 ... 14336;
+//    within 15 % (a few of 65 to 256 rows 29 %). From K = 8192 on (and where
+//    the tiles fill at most an eighth of the CUs) it runs without regard to
+//    whole; at K = 4608 ... 8191 where it is under 0.8 of it, since both fits
+//    are that uncertain there;
+//  * the streaming kernels (w8a8_rows_us): up to 64 rows unless split K from K
+//    = 8192 on is under theirs by 3 %, or, from 49 rows on, over 16384 columns
+//    and K > 4096 the weight rows are not whole 128-byte lines (56 rows of
+//    10048 x 16832 80 us against 69, of 4288 x 17100 37.8 against 35.3; 9472 x
+//    16896 57 against 62); more rows where they are under split K and 0.95 of
+//    whole.
+// Against the choice without the streaming kernels and splits from 8192 on
+// only, 5500 drawn calls (K 1024 ... 14336, N 1024 ... 18944) take 0.46 of the
+// time at 17 to 64 rows, 0.62 at 65 to 256, 0.82 at 257 to 1024 and 0.97 above;
+// 1 % of them are slower by more than 3 %, the worst by 16 %. Streaming all up to 64 rows and
+// comparing tiles with a split fitted to fewer rows was slower on 5 % of 49
+// to 64 rows, by up to half (54 of 12736 x 8512 64 us against 42), and above
+// 1024 rows by up to 1.7 (2049 of 4672 x 1728 62 against 36).
+double split_us(const W8A8Args& a, int64_t tiles, int splits) {
+    const double K = (double)a.width, rows = (double)a.rows, columns = (double)a.columns;
+    return 7.76 + 4.52e-3 * K / splits + 1.41e-6 * splits * rows * columns + 7e-8 * K * columns +
+           5.9e-6 * (double)tiles * K + 0.0154 * (rows < 256.0 ? rows : 256.0);
 }
+
+// room: the workspace holds a split's sums (the size query asks as if it did).
+W8A8Plan plan_w8a8(const W8A8Args& a, bool room) {
+    const int64_t cus = num_cus();
+    const double K = (double)a.width;
+    auto cost = [&](double c, double e, int64_t bm, int64_t bn) {
+        const int64_t tiles = ((a.rows + bm - 1) / bm) * ((a.columns + bn - 1) / bn);
+        const int64_t full = tiles / cus, rem = tiles % cus;
+        const double rounds = (double)full + (rem ? 0.7 + 0.3 * (double)rem / (double)cus : 0.0);
+        return (double)(bm * bn) * (c * K + e) * rounds;
+    };
+    const bool streams = !w8a8_pinned() && w8a8_rows_fits(a);
+    int nb = 0;
+    const double stream_us = streams ? w8a8_rows_us(a.rows, a.columns, a.width, &nb) : 1e30;
+    const W8A8Plan stream{true, nb, 1};
+    if (a.width % 64 != 0 || !ring_offsets_fit(a)) {
+        // Register-staged kernels: any K % 16 == 0.
+        const double c128 = cost(308.0, 250000.0, 256, 128), c192 = cost(280.5, 227212.0, 256, 192);
+        if (streams && (a.rows <= 64 || stream_us / 0.95 < 1.2e-9 * (c128 < c192 ? c128 : c192))) return stream;
+        return {false, c128 < c192 ? 4 : 3, 1};
+    }
+    const int64_t kt = a.width / 64;
+    const int64_t tiles = ((a.rows + 255) / 256) * ((a.columns + 127) / 128);
+    const int sp = room ? w8a8_auto_splits(a.rows, a.columns, a.width, cus) : 1;
+    const double splitting_us = sp > 1 ? split_us(a, tiles, sp) : 1e30;
+    const W8A8Plan split{false, 17, sp};
+    W8A8Plan whole{false, 16, 1};
+    double best = cost(243.7, 117070.0, 256, 192);
+    auto consider = [&](bool ok, double t, int id) {
+        if (ok && t < best) best = t, whole.id = id;
+    };
+    consider(true, cost(281.8, 123726.0, 256, 128), 17);
+    const bool s4 = kt >= 4 && kt % 4 == 0, s3 = kt >= 3 && kt % 3 == 0;
+    // The eight-wave 256 x 256 ring replaces the four-wave one (11), at 0.94
+    // of its fit: measured 0.80-0.92 of its time on seven shapes (4352 x
+    // 12288 -> 3072: 160 against 179 us; 2048 x 4096 -> 14336: 126 against
+    // 139), a factor that keeps 4096 x 3072 -> 12288 and 4096 x 12288 -> 3072
+    // on the 256 x 192 pair ring, which stays faster there.
+    consider(s4, cost(240.7, 163216.0, 256, 256), 19);
+    consider(!s4 && s3, cost(250.7, 210425.0, 256, 256), 14);
+    const double whole_us = 1e-9 * best + 2.5;
+    if (streams && a.rows <= 64) {
+        if (a.rows > 16 && a.width >= 8192 && 0.97 * splitting_us < stream_us) return split;
+        const bool ragged = a.rows > 48 && a.columns > 64 * cus && a.width % 128 != 0 && a.width > 4096;
+        return ragged ? whole : stream;
+    }
+    if (stream_us < splitting_us && stream_us / 0.95 < whole_us) return stream;
+    if (sp > 1 && (w8a8_split_override() > 1 || a.width >= 8192 || 8 * tiles <= cus || splitting_us < 0.8 * whole_us))
+        return split;
+    return whole;
+}
+
+}  // namespace
 
 int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width) {
     if (rows <= 0 || columns <= 0 || width % 64 != 0) return 0;
@@ -1521,11 +1614,8 @@ int64_t w8a8_partial_elems(int64_t rows, int64_t columns, int64_t width) {
     a.columns = columns;
     a.width = width;
     if (!ring_offsets_fit(a)) return 0;
-    const int sp = w8a8_auto_splits(rows, columns, width, num_cus());
-    if (sp > 1 && !w8a8_pinned() && w8a8_rows_fits(a)) {  // the streaming kernels need none
-        int nb;
-        if (rows <= 64 || tiles_beat_split(a, w8a8_rows_us(rows, columns, width, &nb))) return 0;
-    }
+    const int sp = w8a8_tile_override() != 0 ? w8a8_auto_splits(rows, columns, width, num_cus())
+                                             : plan_w8a8(a, true).splits;
     return sp > 1 ? (int64_t)sp * rows * columns : 0;
 }
 
@@ -1550,76 +1640,17 @@ hipError_t launch_w8a8_mfma(const W8A8Args& a, hipStream_t stream) {
             break;
         default: break;
     }
-    const bool pinned = w8a8_pinned();
-    // Up to 64 rows the weights' stream is all that counts: on every shape
-    // measured (rows.hip) the streaming kernel is ahead of 256-row tiles.
-    if (!pinned && a.rows <= 64 && w8a8_rows_fits(a)) return launch_w8a8_rows(a, 0, stream);
-    // Cost model, fitted to MI355X timings of every candidate on ten shapes
-    // (the BASELINE GEMM shapes and the reference's 256-row benchmark shapes;
-    // codes of N(0,1) rows and uniform weights rotated past the MALL, f32
-    // out): a kernel runs its
-    // tiles in rounds of one tile per CU, a round costs BM * BN * (c * K + e)
-    // (c: per output element and K byte; e: the per-tile prologue and
-    // epilogue), and a partial last round with fill f costs (0.7 + 0.3 f) of
-    // a full one (the chip is power-limited on this path, so a partly idle
-    // round runs at a higher clock). It picks the fastest candidate, or one
-    // within 1 %, on all ten operands rotated; the other kernels
-    // (register-staged, two-waves-per-SIMD DMA, single-refill rings at
-    // 256 x 192 and 256 x 128) lost on every one and stay reachable through
-    // OMNI_W8A8_TILE.
-    const int64_t cus = num_cus();
-    const double K = (double)a.width;
-    auto cost = [&](double c, double e, int64_t bm, int64_t bn) {
-        const int64_t tiles = ((a.rows + bm - 1) / bm) * ((a.columns + bn - 1) / bn);
-        const int64_t full = tiles / cus, rem = tiles % cus;
-        const double rounds = (double)full + (rem ? 0.7 + 0.3 * (double)rem / (double)cus : 0.0);
-        return (double)(bm * bn) * (c * K + e) * rounds;
-    };
-    struct Cand { double t; int id; };
-    // More rows on small matrices: the streaming kernels' tiles, where their
-    // time by w8a8_rows_us is below 0.95 of the choice below. That choice's
-    // time, fitted to 78 timings (65 to 1024 rows, thirteen K x N of 1152 ...
-    // 14336 x 1152 ... 28672) where its tiles leave CUs idle: the cost model's
-    // (in fs) plus 2.5 us unsplit, 1.2 times it for the register-staged
-    // kernels, and for split K and its reduction a line in the weights' MB
-    // and the rows. On 117 timings (those shapes at 65 to 1024 rows) the rule's
-    // choice is within 6 % of the fastest on 107 and 18 % off at worst; the
-    // tiles are up to 5 times faster (65 rows of 4304 x 1152).
-    int tiles_nb = 0;
-    const double tiles_us =
-        !pinned && w8a8_rows_fits(a) ? w8a8_rows_us(a.rows, a.columns, a.width, &tiles_nb) / 0.95 : 1e30;
-    if (a.width % 64 != 0 || !ring_offsets_fit(a)) {
-        // Register-staged kernels: any K % 16 == 0.
-        const double c128 = cost(308.0, 250000.0, 256, 128), c192 = cost(280.5, 227212.0, 256, 192);
-        if (tiles_us < 1.2e-9 * (c128 < c192 ? c128 : c192)) return launch_w8a8_rows(a, tiles_nb, stream);
-        return cost(308.0, 250000.0, 256, 128) < cost(280.5, 227212.0, 256, 192) ? launch_bn<128, 2>(a, stream)
-                                                                                 : launch_bn<192, 2>(a, stream);
-    }
-    const int64_t kt = a.width / 64;
-    const int sp = w8a8_auto_splits(a.rows, a.columns, a.width, cus);
-    if (sp > 1) {
-        if (tiles_beat_split(a, 0.95 * tiles_us)) return launch_w8a8_rows(a, tiles_nb, stream);
-        const int64_t tiles = ((a.rows + 255) / 256) * ((a.columns + 127) / 128);
-        if (fit_splits(a, tiles, (int)kt, sp) > 1) return launch_pair<128>(a, stream, sp);
-    }
-    Cand best{cost(243.7, 117070.0, 256, 192), 16};
-    auto consider = [&](bool ok, double t, int id) {
-        if (ok && t < best.t) best = Cand{t, id};
-    };
-    consider(true, cost(281.8, 123726.0, 256, 128), 17);
-    const bool s4 = kt >= 4 && kt % 4 == 0, s3 = kt >= 3 && kt % 3 == 0;
-    // The eight-wave 256 x 256 ring replaces the four-wave one (11), at 0.94
-    // of its fit: measured 0.80-0.92 of its time on seven shapes (config 4's
-    // MLP down 4352 x 12288 -> 3072: 160 against 179 us; config 3's 2048 x
-    // 4096 -> 14336: 126 against 139), a factor that keeps both north-star
-    // shapes on the 256 x 192 pair ring, which stays faster there.
-    consider(s4, cost(240.7, 163216.0, 256, 256), 19);
-    consider(!s4 && s3, cost(250.7, 210425.0, 256, 256), 14);
-    if (tiles_us < 1e-9 * best.t + 2.5) return launch_w8a8_rows(a, tiles_nb, stream);
-    switch (best.id) {
+    // Whether the workspace holds the sums of the split K that would run.
+    const int64_t tiles = ((a.rows + 255) / 256) * ((a.columns + 127) / 128);
+    const int sp = w8a8_auto_splits(a.rows, a.columns, a.width, num_cus());
+    const W8A8Plan plan = plan_w8a8(a, sp > 1 && fit_splits(a, tiles, (int)(a.width / 64), sp) > 1);
+    if (plan.stream) return launch_w8a8_rows(a, plan.id, stream);
+    switch (plan.id) {
         case 19: return launch_ring8_256(a, stream);
         case 14: return launch_ring<256, 3>(a, stream);
-        case 17: return launch_pair<128>(a, stream);
+        case 17: return launch_pair<128>(a, stream, plan.splits);
+        case 4: return launch_bn<128, 2>(a, stream);
+        case 3: return launch_bn<192, 2>(a, stream);
         default: return launch_pair<192>(a, stream);
     }
 }

@@ -110,6 +110,17 @@ def test_tuning_knobs_set_unset_restore():
     assert L.omni_int8_set_tuning(None, 2, 1) == _lib.OMNI_BAD_ARGUMENT
 
 
+@pytest.mark.parametrize("rows,columns,width,splits", [
+    (16, 8512, 12736, 0), (54, 8512, 12736, 3), (44, 9152, 11328, 3), (62, 2040, 12736, 6), (64, 1536, 8960, 0),
+    (64, 8192, 8128, 0), (64, 4096, 8208, 0), (1577, 1280, 9920, 3), (256, 4096, 12288, 0), (512, 4096, 12288, 4),
+    (2049, 1728, 4672, 0)])
+def test_w8a8_streams_only_where_split_k_is_slower(rows, columns, width, splits):
+    # W8A8 routes are bit-identical; the size query tells split K apart. Long K
+    # over columns that leave the streaming kernel a nearly empty last round,
+    # or many rows, split (256 CUs, as without a device).
+    assert _lib.lib().omni_w8a8_gemm_workspace_size(rows, columns, width) == splits * rows * columns * 4
+
+
 @pytest.mark.parametrize("rows,columns,width", [(8, 4096, 4096), (64, 1536, 8960), (256, 4096, 12288)])
 def test_a_pinned_w8a8_split_is_honoured(knobs, rows, columns, width):
     # OMNI_W8A8_SPLITS forces split K, also where the streaming kernels
