@@ -589,14 +589,25 @@ double w8a8_rows_us(int64_t rows, int64_t columns, int64_t width, int* nb) {
 //    of 2048 x 7168 5.45 against 5.55, 8 even; 5 of 3072 x 4112 7.3 against
 //    5.9);
 //  * three and four rows, the GEMV up to K = 4096 on up to 8192 columns (4 of
-//    4096 x 4096 5.8 against 6.1, 3 of 5120 x 5120 9.0 against 9.4) and at K =
-//    4096 up to 64 M weights (4 of 4096 x 14336 13.9 against 14.5; beyond, 4
-//    of 4096 x 28672 22.8 against 24.1, of 14336 x 4096 12.6 against 15.3);
+//    4096 x 4096 5.8 against 6.1, 3 of 5120 x 5120 9.0 against 9.4), up to K =
+//    8192 on up to 2048 (3 of 7616 x 1344 5.4 against 6.8, 4 of 8192 x 2048 5.8
+//    against 6.4) and at K = 4096 up to 64 M weights (4 of 4096 x 14336 13.9
+//    against 14.5; beyond, 4 of 4096 x 28672 22.8 against 24.1, of 14336 x 4096
+//    12.6 against 15.3); and where weight rows start within 64-byte pieces, which
+//    the copies then straddle (4 of 4064 x 12736 13.4 against 15.5, of 5456 x
+//    1928 5.5 against 6.6, of 11536 x 2176 10.4 against 11.4);
+//  * 17 to 32 rows of long K, the GEMM where blocks of 32 columns leave a nearly
+//    empty second round: 25 rows and more from K = 8300 on (32 of 12160 x 10048
+//    44 against 48 us, 31 of 9856 x 9088 33 against 37), and where weight rows
+//    are not whole 128-byte lines from K = 5300 (30 of 6080 x 8576 24 against
+//    27, of 13760 x 9200 45 against 59), up to 24 from 8000 (20 of 10432 x 8832
+//    35.5 against 39.5, 23 of 8128 x 8320 28 against 33);
 //  * from 33 rows on, the GEMM where the matrix is large: each activation
 //    copy is then read by too few columns (48 of 4096 x 14336 28.3 against
 //    25.8 us, but of 4096 x 6144 15.1 against 29.2, of 14336 x 4096 29.9
-//    against 32.8; 64 of 2048 x 14336 18.6 against 17.4, of 4096 x 5120 15.7
-//    against 17.5, of 8960 x 1536 24.4 against 37.1).
+//    against 32.8; 36 of 1984 x 16960 19.5 against 17.4; 64 of 2048 x 14336
+//    18.6 against 17.4, of 4096 x 5120 15.7 against 17.5, of 8960 x 1536 24.4
+//    against 37.1; 50 of 1088 x 18240 15.3 against 12.2).
 bool w8a16_rows_take(const W8A16Args& a) {
     if (a.rows > 64 || a.width % 16 != 0 || a.width < 16 || a.width > kMaxRowBytes) return false;
     const int64_t cus = num_cus();
@@ -605,17 +616,21 @@ bool w8a16_rows_take(const W8A16Args& a) {
     if (a.width > 16384 && a.rows <= 4) return true;
     if (a.rows <= 2) return false;
     if (a.rows <= 4) {
-        if (a.width == 4096 && elems <= (64 << 20)) return false;
-        return wide ? a.columns >= 8192 : a.width > 4096;
+        if (a.width % 64 != 0 || (a.width == 4096 && elems <= (64 << 20))) return false;
+        return wide ? a.columns >= 8192 : a.width > 8192 || (a.width > 4096 && a.columns > 8 * cus);
     }
     if (a.rows <= 16) {
         if (a.width > 4096 || a.width % 1024 != 0) return true;
         if (a.width == 1024) return a.columns > (a.rows <= 8 ? 32 : 17) * cus;
         return a.width == 2048 && a.rows < 8 ? a.columns >= 32 * cus : wide;
     }
-    if (a.rows <= 32) return true;
-    if (a.rows <= 48) return !wide || elems <= 36e6;
-    return elems < 16e6 || (a.width <= 4096 && elems <= 26e6);
+    if (a.rows <= 32) {
+        if (a.columns <= 32 * cus || a.columns > 42 * cus || a.width % 64 != 0) return true;  // (K % 64: no ring)
+        if (a.width % 128 == 0) return a.rows <= 24 || a.width < 8300;
+        return a.width < (a.rows <= 24 ? 8000 : 5300);
+    }
+    if (a.rows <= 48) return !wide || elems <= (a.columns > 64 * cus ? 32e6 : 36e6);
+    return elems < 16e6 || (a.width <= 4096 && a.columns <= 64 * cus && elems <= 26e6);
 }
 
 hipError_t launch_w8a16_rows(const W8A16Args& w, hipStream_t st) {

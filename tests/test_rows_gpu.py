@@ -154,23 +154,35 @@ def test_w4a16_stream_scales(rows, width, columns, low, high):
     assert fits.any() and (np.abs(got - exact) <= bound)[fits].all()
 
 
-# Just past one round of its workgroups the LDS skinny kernel (route 1) keeps a
-# few rows of short K; elsewhere the streaming kernel's sums, in another order,
-# differ in some output's last bit.
-@pytest.mark.parametrize("rows,width,columns,skinny", [
-    (5, 1024, 4096, True), (5, 1024, 4112, True), (8, 1024, 8192, True), (8, 1024, 8208, False),
-    (16, 1024, 4352, True), (16, 1024, 4368, False), (7, 2048, 8176, True), (7, 2048, 8192, False),
-    (8, 2048, 4112, False), (5, 3072, 4112, False), (5, 1040, 4096, False)])
-def test_w8a16_short_k_past_one_round(rows, width, columns, skinny, knobs):
+# Where the routes part. Route 1 pins the GEMV (up to 4 rows) or the skinny
+# kernel, 2 the GEMM; the streaming kernel's sums, in another order than either's,
+# differ in some output's last bit (0).
+@pytest.mark.parametrize("rows,width,columns,route", [
+    (5, 1024, 4096, 1), (5, 1024, 4112, 1), (8, 1024, 8192, 1), (8, 1024, 8208, 0), (16, 1024, 4352, 1),
+    (16, 1024, 4368, 0), (7, 2048, 8176, 1), (7, 2048, 8192, 0), (8, 2048, 4112, 0), (5, 3072, 4112, 0),
+    (5, 1040, 4096, 0),
+    (3, 7808, 1408, 1), (4, 8192, 2048, 1), (4, 8192, 2064, 0), (4, 8256, 2048, 0), (4, 8272, 2048, 1),
+    (4, 4064, 12736, 1), (4, 4160, 12736, 0), (4, 16400, 3000, 0),
+    (30, 13760, 9200, 2), (30, 13760, 8192, 0), (30, 13760, 10768, 0), (25, 11904, 9152, 2), (24, 11904, 9152, 0),
+    (25, 8192, 9152, 0), (25, 11904, 10752, 2), (31, 5312, 8252, 2), (31, 5184, 8252, 0), (20, 8000, 9728, 2),
+    (20, 7872, 9728, 0), (30, 14064, 8576, 0), (36, 1984, 16960, 2), (36, 1920, 16384, 0),
+    (50, 1088, 18240, 2), (50, 1088, 14656, 0)])
+def test_w8a16_routes(rows, width, columns, route, knobs):
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the columns are those of 256 CUs")
     g = torch.Generator(device="cuda").manual_seed(rows + width + columns)
     x = torch.randn((rows, width), generator=g, device="cuda").half()
     w = torch.randint(-127, 128, (columns, width), generator=g, device="cuda", dtype=torch.int8)
     scale = torch.rand(columns, generator=g, device="cuda").half()
-    got = oi.w8a16_linear(x, w, scale)
-    knobs.set("OMNI_W8A16_ROUTE", "1")
-    assert torch.equal(got, oi.w8a16_linear(x, w, scale)) == skinny
+    routes_agree(lambda: oi.w8a16_linear(x, w, scale), route, knobs)
+
+
+def routes_agree(call, route, knobs):
+    got = call()
+    for pin in ("1", "2"):
+        knobs.set("OMNI_W8A16_ROUTE", pin)
+        if route in (0, int(pin)):
+            assert torch.equal(got, call()) == (route != 0), pin
 
 
 # A knob at its automatic value leaves the choice as it is without the knob; a
