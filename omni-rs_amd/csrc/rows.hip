@@ -666,23 +666,38 @@ hipError_t launch_w8a16_rows(const W8A16Args& w, hipStream_t st) {
 // GEMM:
 // 4 rows of 4096 x 6144 6.8 against 8.7 us, of 3584 x 18944 13.2 against
 // 15.9, 8 of 4096 x 14336 12.2 against 21.6, 16 of 14336 x 4096 16.2 against
-// 28.9, 32 of 3584 x 18944 29.8 against 40.3. The GEMV keeps three and four
-// rows of narrow long-K matrices (4 of 8960 x 1536 7.4 against 7.8); one and
-// two rows of K > 32768 are past its limit. 48 rows of 4096 x 6144 12.5 against
-// 32.2 us, of 8192 x 28672 80 against 93; from 49 rows on, in blocks of 16
-// columns (64 of 8960 x 1536 21.2 against 37.9, of 2048 x 8192 12.6 against
-// 18.3, of 4096 x 6144 19.4 against 20.6), the GEMM keeps what is wide and large
-// (64 of 4096 x 14336 36.0 against 30.0) or very wide (of 1024 x 18944 16.4
-// against 14.8).
+// 28.9, 32 of 3584 x 18944 29.8 against 40.3. The others keep:
+//  * three and four rows, the GEMV on narrow matrices of long K (4 of 8960 x
+//    1536 7.4 against 7.8; below 1408 columns 3 of 2432 x 1088 3.85 against
+//    4.04); one and two rows of K > 32768 are past its limit;
+//  * where weight rows are not whole 128-byte lines (K % 256 != 0), which the
+//    copies then straddle: three and four rows in a nearly empty second round of
+//    32-column blocks, the GEMV (4 of 7040 x 9216 15.3 against 17.8, 3 of 4480 x
+//    10112 11.9 against 13.4); some rows of short K, the skinny kernel, whose
+//    loads split K evenly over more waves (9 of 1152 x 8488 6.2 against 7.4, 17
+//    of 1152 x 1792 4.13 against 4.50, 9 of 2176 x 2200 4.40 against 4.84);
+//  * from 49 rows on (in blocks of 16 columns: 64 of 8960 x 1536 21.2 against
+//    37.9, of 2048 x 8192 12.6 against 18.3, of 4096 x 6144 19.4 against 20.6),
+//    the GEMM, what is wide and large (64 of 4096 x 14336 36.0 against 30.0; 61
+//    of 5632 x 4416 25.8 against 23.3) or very wide (of 1024 x 18944 16.4
+//    against 14.8). 48 rows of 4096 x 6144 12.5 against 32.2, of 8192 x 28672
+//    80 against 93.
 bool w4a16_rows_take(const W8A16Args& a) {
     if (a.rows > 64 || a.group != kInt4Group || a.width % kInt4Group != 0 || a.width <= 0 || a.width > kMaxRowBytes)
         return false;
+    const int64_t cus = num_cus();
+    const bool wide = is_wide(a.columns, cus), lines = a.width % 256 == 0;
+    const bool second_round = a.columns > 32 * cus && a.columns <= 44 * cus;
     if (a.width > 32768 && a.rows <= 4) return true;
     if (a.rows <= 2) return false;
-    if (a.rows <= 4) return a.columns > 2048 || a.width <= 4096;
-    const int64_t cus = num_cus();
-    return a.rows <= 48 || !is_wide(a.columns, cus) ||
-           (a.columns <= 40 * cus && (double)a.columns * (double)a.width <= 26e6);
+    if (a.rows <= 4) {
+        if (!lines && second_round && a.width >= 4096) return false;
+        return a.columns > 2048 || (a.width <= 4096 && a.columns >= 1408);
+    }
+    if (!lines && a.rows > 8 && a.rows <= 24 && a.width < 1280 && (!wide || second_round)) return false;
+    if (!lines && a.rows > 8 && a.rows <= 12 && a.width > 2048 && a.width < 3584 && !wide) return false;
+    return a.rows <= 48 || !wide ||
+           (a.columns <= 40 * cus && (double)a.columns * (double)a.width <= (a.width <= 4096 ? 26e6 : 22e6));
 }
 
 hipError_t launch_w4a16_rows(const W8A16Args& w, hipStream_t st) {

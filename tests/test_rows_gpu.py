@@ -120,8 +120,16 @@ def w8a16_case(rows, width, columns):
     (5, 256, 15), (8, 1792, 100), (7, 768, 4100), (9, 3328, 17), (16, 256, 64), (13, 1280, 4097), (17, 512, 31),
     (32, 2816, 70), (29, 768, 4129), (6, 256, 131100), (5, 128, 33), (8, 1152, 100), (16, 2944, 4099), (3, 4224, 2051),
     (32, 1408, 65), (17, 384, 4130), (33, 128, 47), (48, 640, 4100), (40, 1408, 130), (47, 256, 131104),
-    (49, 256, 33), (64, 1152, 70), (63, 384, 4099), (56, 128, 131100)])
+    (49, 256, 33), (64, 1152, 70), (63, 384, 4099)])
 def test_w4a16_stream(oracle, rows, width, columns):
+    w4a16_case(rows, width, columns)
+
+
+def test_w4a16_very_wide():  # the GEMM, whose tiles outnumber the CUs four times
+    w4a16_case(56, 128, 131100)
+
+
+def w4a16_case(rows, width, columns):
     rng = np.random.default_rng(rows + 5 * width + columns)
     x = rng.standard_normal((rows, width)).astype(np.float16)
     packed = rng.integers(0, 256, (columns, width // 2), dtype=np.uint8)
@@ -175,6 +183,23 @@ def test_w8a16_routes(rows, width, columns, route, knobs):
     w = torch.randint(-127, 128, (columns, width), generator=g, device="cuda", dtype=torch.int8)
     scale = torch.rand(columns, generator=g, device="cuda").half()
     routes_agree(lambda: oi.w8a16_linear(x, w, scale), route, knobs)
+
+
+@pytest.mark.parametrize("rows,width,columns,route", [
+    (4, 7040, 9216, 1), (4, 7168, 9216, 0), (4, 7040, 8192, 0), (4, 7040, 11280, 0), (3, 2432, 1392, 1),
+    (3, 2432, 1408, 0), (4, 4352, 2048, 1), (4, 4352, 2064, 0),
+    (9, 1152, 8488, 1), (8, 1152, 8488, 0), (24, 1152, 4096, 1), (25, 1152, 4096, 0), (17, 1152, 4112, 0),
+    (17, 1280, 2048, 0), (12, 2176, 2200, 1), (13, 2176, 2200, 0), (9, 2304, 2200, 0), (9, 3456, 4096, 1),
+    (9, 3712, 4096, 0),
+    (61, 5632, 4416, 2), (61, 4096, 4416, 0)])
+def test_w4a16_routes(rows, width, columns, route, knobs):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the columns are those of 256 CUs")
+    g = torch.Generator(device="cuda").manual_seed(rows + width + columns)
+    x = torch.randn((rows, width), generator=g, device="cuda").half()
+    w = torch.randint(0, 256, (columns, width // 2), generator=g, device="cuda", dtype=torch.uint8)
+    scale = torch.rand((columns, width // 128), generator=g, device="cuda").bfloat16()
+    routes_agree(lambda: oi.w4a16_linear(x, w, scale), route, knobs)
 
 
 def routes_agree(call, route, knobs):
