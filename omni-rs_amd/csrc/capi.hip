@@ -134,7 +134,9 @@ bool w4a16_pinned() {
 // GEMM once per 64 to 256, so the GEMM wins on big matrices (MI355X, W8A16
 // 4096 -> 14336: 24.5 against 37.7 us at 24 rows, 27.4 against 70.5 at 64;
 // 4096 -> 4096 stays skinny to 48 rows: 15.5 against 16.8). W4A16 over a
-// long K (14336 -> 4096) stays skinny to 48 rows (40.3 against 43.4 at 32).
+// long K (14336 -> 4096) stays skinny to 48 rows (40.3 against 43.4 at 32);
+// over very many columns it leaves it from 49 on (1024 -> 12288 15.6 against
+// 17.2 at 56, 1024 -> 15360 17.1 against 22.5).
 // Those GEMM times are the ring kernels'. Where no ring can run (K % 64 !=
 // 0 and the like) the register-staged GEMM takes only more than 48 rows of
 // at least 32 M weights (W8A16 K = 4112: 48 x 9000 39.2 us skinny against
@@ -142,7 +144,7 @@ bool w4a16_pinned() {
 bool midrows_take_gemm(int64_t rows, int64_t columns, int64_t width, bool int4, bool ring_ok) {
     const double elems = (double)columns * (double)width;
     if (!ring_ok) return rows > 48 && elems >= 32e6;
-    if (rows > 48 && elems >= 16e6) return true;
+    if (rows > 48 && (elems >= 16e6 || (int4 && columns > 40 * omni::num_cus()))) return true;
     if (int4 && columns < 2 * width) return false;
     return elems >= 32e6;
 }

@@ -191,7 +191,7 @@ def test_w8a16_routes(rows, width, columns, route, knobs):
     (9, 1152, 8488, 1), (8, 1152, 8488, 0), (24, 1152, 4096, 1), (25, 1152, 4096, 0), (17, 1152, 4112, 0),
     (17, 1280, 2048, 0), (12, 2176, 2200, 1), (13, 2176, 2200, 0), (9, 2304, 2200, 0), (9, 3456, 4096, 1),
     (9, 3712, 4096, 0),
-    (61, 5632, 4416, 2), (61, 4096, 4416, 0)])
+    (61, 5632, 4416, 2), (61, 4096, 4416, 0), (56, 1024, 12288, 2), (56, 1024, 10240, 0), (48, 1024, 12288, 0)])
 def test_w4a16_routes(rows, width, columns, route, knobs):
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the columns are those of 256 CUs")
