@@ -7,7 +7,10 @@ or fails to load, every call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
+import types
+import warnings
 
 OMNI_OK = 0
 OMNI_NOT_HANDLED = 1
@@ -26,6 +29,11 @@ OMNI_LOWERING_SCALAR = 2
 # host-sanitised one that tests/sanitize_cpu.sh runs the CPU tests on).
 LIB_PATH = os.environ.get("OMNI_INT8_LIBRARY") or os.path.join(
     os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "libomni_int8.so")
+
+# The direct calls' module, and likewise another build of it.
+HOST_PATH = os.environ.get("OMNI_INT8_HOST") or os.path.join(os.path.dirname(os.path.abspath(__file__)), "_host.so")
+HOST_CALLS = ("try_int8_gemm", "convrot_linear", "quantize_rows", "w8a8_gemm", "w8a16_linear", "w4a16_linear",
+              "f16_linear")
 
 # name -> (restype, argtypes); one entry per declaration in include/omni_int8.h
 _P = ctypes.c_void_p
@@ -98,18 +106,28 @@ def check(status: int) -> int:
     return status
 
 
+def _load_host():
+    spec = importlib.util.spec_from_file_location(f"{__package__}._host", HOST_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
 def host():
     """The package's direct calls (csrc/host.cpp, built beside the library),
     bound to the same library as lib(). Each returns NotImplemented where its
-    Python wrapper has to do the work."""
+    Python wrapper has to do the work; where the module is not there or does
+    not load, all do, and calls cost the wrappers' host time."""
     global _host
     if _host is None:
-        try:
-            from . import _host as module
-        except ImportError as e:
-            raise OmniError(OMNI_BAD_ARGUMENT,
-                            f"omni_int8/_host.so does not load ({e}); build it with `make -C omni-rs_amd`") from None
         handle = lib()
-        module.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in SIGNATURES})
+        try:
+            module = _load_host()
+        except ImportError as e:
+            warnings.warn(f"{HOST_PATH} does not load ({e}): calls go through the Python wrappers, which take 3 to 9 us "
+                          "more each; build it with `make -C omni-rs_amd`", RuntimeWarning, stacklevel=3)
+            module = types.SimpleNamespace(**{name: lambda *args: NotImplemented for name in HOST_CALLS})
+        else:
+            module.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in SIGNATURES})
         _host = module
     return _host

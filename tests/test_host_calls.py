@@ -2,6 +2,7 @@
 for: the same results for every form of argument, and NotImplemented wherever
 the wrapper has to do the work."""
 import threading
+import warnings
 
 import pytest
 import torch
@@ -144,6 +145,38 @@ def test_direct_calls_from_threads_and_streams():
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+@pytest.mark.parametrize("content", [None, b"not a shared object"])
+def test_calls_work_without_the_module(content, tmp_path, monkeypatch):
+    # The library alone is enough, as it was before the direct calls: a module
+    # that is missing or does not load is said once, and the wrappers do the work.
+    path = tmp_path / "_host.so"
+    if content:
+        path.write_bytes(content)
+    monkeypatch.setattr(_lib, "HOST_PATH", str(path))
+    monkeypatch.setattr(_lib, "_host", None)
+    x, w = torch.zeros((2, 64)).half(), torch.zeros((64, 8)).half()
+    with pytest.warns(RuntimeWarning, match="does not load"):
+        assert f16.depth_try_linear(x, w) is None  # host tensors
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert f16.depth_try_linear(x, w) is None
+        with pytest.raises(oi.OmniError):
+            oi.quantize_rows(x)
+    assert all(getattr(_lib.host(), name)() is NotImplemented for name in _lib.HOST_CALLS)
+
+
+@pytest.mark.gpu
+def test_calls_run_without_the_module(tmp_path, monkeypatch):
+    every = calls("cuda")
+    want = {k: f() for k, f in every.items()}
+    monkeypatch.setattr(_lib, "HOST_PATH", str(tmp_path / "_host.so"))
+    monkeypatch.setattr(_lib, "_host", None)
+    with pytest.warns(RuntimeWarning, match="does not load"):
+        got = {k: f() for k, f in every.items()}
+    for k in every:
+        same(got[k], want[k])
 
 
 def test_direct_calls_leave_host_tensors_to_the_wrapper():
