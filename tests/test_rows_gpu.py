@@ -80,13 +80,14 @@ def close(got, want):
     assert tolerance.rel_err(host(got), want) <= tolerance.FP16_REL_TOL
 
 
-# Shapes that the streaming kernels take by default (w8a16_rows_take): every
-# row block, K % 64 and K % 256 not 0, one block and several per workgroup.
+# Shapes that the streaming kernels take by default (w8a16_rows_take; three and
+# four rows of K % 64 != 0 the GEMV): every row block, K % 64 and K % 256 not 0,
+# one block and several per workgroup.
 @pytest.mark.parametrize("rows,width,columns", [
     (1, 18944, 40), (4, 16400, 33), (3, 4112, 17), (4, 1552, 8195), (5, 16, 7), (6, 1040, 100), (8, 4624, 4100),
     (8, 1168, 4112), (9, 4112, 64), (16, 240, 31), (13, 4096, 4113), (16, 528, 9000), (17, 64, 16), (32, 1104, 50),
     (31, 336, 4130), (33, 272, 40), (48, 1040, 300), (47, 368, 4100), (49, 144, 30), (64, 2064, 70), (63, 400, 4101),
-    (24, 32, 131200)])
+    (24, 32, 131200), (3, 8256, 17), (4, 1600, 8195), (4, 4160, 2100)])
 def test_w8a16_stream(rows, width, columns):
     w8a16_case(rows, width, columns)
 
@@ -108,11 +109,14 @@ def w8a16_case(rows, width, columns):
     exact = (x.astype(np.float64) @ w.T.astype(np.float64)) * scale.astype(np.float64)
     close(oi.w8a16_linear(dev(x), dev(w), dev(scale)), exact)
     close(oi.w8a16_linear(dev(x), dev(w), dev(scale), dev(bias)), exact + bias.astype(np.float64))
-    # a row's infinity stays in its row
-    x[0, width - 1] = np.inf
-    got = host(oi.w8a16_linear(dev(x), dev(w), dev(scale)))
-    assert not np.isfinite(got[0]).any() or (w[:, -1] == 0).any()
-    assert np.isfinite(got[1:]).all()
+    # a row's infinity stays in its row (times a weight of 0 it is NaN), also in
+    # the last one, which the kernels' row blocks repeat
+    for row in {0, rows - 1}:
+        y = x.copy()
+        y[row, width - 1] = np.inf
+        got = host(oi.w8a16_linear(dev(y), dev(w), dev(scale)))
+        assert not np.isfinite(got[row]).any()
+        assert np.isfinite(np.delete(got, row, 0)).all()
 
 
 @pytest.mark.parametrize("rows,width,columns", [
@@ -120,7 +124,7 @@ def w8a16_case(rows, width, columns):
     (5, 256, 15), (8, 1792, 100), (7, 768, 4100), (9, 3328, 17), (16, 256, 64), (13, 1280, 4097), (17, 512, 31),
     (32, 2816, 70), (29, 768, 4129), (6, 256, 131100), (5, 128, 33), (8, 1152, 100), (16, 2944, 4099), (3, 4224, 2051),
     (32, 1408, 65), (17, 384, 4130), (33, 128, 47), (48, 640, 4100), (40, 1408, 130), (47, 256, 131104),
-    (49, 256, 33), (64, 1152, 70), (63, 384, 4099)])
+    (49, 256, 33), (64, 1152, 70), (63, 384, 4099), (3, 256, 1411), (4, 2304, 1409)])
 def test_w4a16_stream(oracle, rows, width, columns):
     w4a16_case(rows, width, columns)
 
@@ -147,7 +151,7 @@ def w4a16_case(rows, width, columns):
 @pytest.mark.parametrize("low,high", [(1e-6, 5e-5), (8192.0, 65536.0)])
 @pytest.mark.parametrize("rows,width,columns", [
     (3, 256, 2100), (4, 640, 33), (8, 384, 100), (16, 512, 4200), (32, 128, 70),
-    (48, 384, 40), (64, 256, 4100)])
+    (48, 384, 40), (64, 256, 4100), (4, 640, 1411)])
 def test_w4a16_stream_scales(rows, width, columns, low, high):
     rng = np.random.default_rng(rows + width + columns)
     x = (rng.standard_normal((rows, width)) * (1.0 if high < 1 else 2e-3)).astype(np.float16)

@@ -148,9 +148,8 @@ def test_ring_integer_inputs_are_exact(monkeypatch, tile, knobs):
 
 @pytest.mark.parametrize("tile", ["0", "4", "18"])
 def test_scales_at_an_odd_bf16_offset(oracle, monkeypatch, tile, knobs):
-    # The rings copy scales as 4-byte pairs; a scale array starting 2 bytes
-    # past a 4-byte boundary (a contiguous view at an odd element) takes the
-    # register-staged kernel instead, with the same result bar
+    # The rings copy scales two bytes at a time, so a scale array may start 2
+    # bytes past a 4-byte boundary (a contiguous view at an odd element)
     knobs.set("OMNI_W4A16_TILE", tile)
     rng = np.random.default_rng(int(tile) + 11)
     x, packed, bits, b = wd.random_case(rng, 300, 1024, 200, 128, bias=True)
