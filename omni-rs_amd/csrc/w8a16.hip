@@ -2002,12 +2002,13 @@ int w8a16_tile_override() { return knob(Knob::W8A16Tile, 0); }
 // two or three workgroups per CU the busiest CU's share of them past the
 // first), a launch t0, and a split's reduction r0 + r1 us per million of its
 // partial sums.
-// unsplit and split weigh the estimate where its error has a sign. r0 = 0: not
-// split.
+// unsplit and split weigh the estimate where its error has a sign, later also
+// an unsplit one of more than one round that ends in a partial one. r0 = 0:
+// not split.
 struct RingFit {
     int id;  // as OMNI_W8A16_TILE and OMNI_W4A16_TILE number the rings
     int bm, bn, occ;
-    double a, b, p, t0, r0, r1, unsplit, split;
+    double a, b, p, t0, r0, r1, unsplit, split, later = 1.0;
 };
 struct RingChoice {
     int id, splits;
@@ -2030,7 +2031,7 @@ RingChoice pick_ring(const RingFit* fits, size_t count, const W8A16Args& a, int 
                                            : (double)((rem + cus - 1) / cus - 1) / (double)(f.occ - 1);
             const double rounds = (double)full + (rem ? f.p + (1.0 - f.p) * fill : 0.0);
             double t = f.t0 + rounds * (f.a + 1e-3 * f.b * (double)a.width / sp);
-            if (sp == 1) return t * f.unsplit;
+            if (sp == 1) return t * f.unsplit * (full && rem ? f.later : 1.0);
             return (t + f.r0 + 1e-6 * f.r1 * sp * (double)a.rows * (double)a.columns) * f.split;
         };
         auto splits = [&](int sp) {  // every split non-empty, and room for its sums
@@ -2075,19 +2076,24 @@ W16Plan plan_w8a16(const W8A16Args& a, int cus, bool ws_limited) {
     // off: 582 x 7680 -> 3264 41 us against 69 (128 x 192 tiles split three
     // ways), 109 x 3968 -> 2112 14 against 22. 192 x 256 tiles fill the rounds
     // that 128 x 320 and 256 x 256 leave ragged: 2550 x 1152 -> 8064 55 us
-    // against 63, 159 x 11008 -> 17920 83 (split three ways) against 107.
+    // against 63, 159 x 11008 -> 17920 83 (split three ways) against 107. The
+    // weights of the last three columns from 3400 further calls: past one round
+    // 128 x 128 tiles two per CU and 192 x 256 ones take 1.15 and 1.3 times
+    // their fit (3565 x 9280 -> 4824 372 against 330 in 128 x 320, 1961 x 1664
+    // -> 9472 88 against 76). Against those rules 0.94 of the time, slower by
+    // more than 3 % on 1 %, by more than 8 % on 0.3 %.
     static constexpr RingFit kFits[] = {
         {5, 128, 128, 1, 4.67, 7.53, 0.69, 1.97, 0.0, 0.00, 1.08, 1.00},
         {8, 64, 128, 1, 2.63, 5.39, 0.83, 2.13, 0.0, 0.00, 1.00, 1.00},
         {9, 256, 192, 1, 10.32, 17.21, 0.73, 4.28, 1.3, 0.81, 1.00, 1.00},
-        {10, 128, 128, 2, 0.71, 13.57, 0.45, 5.10, 2.4, 1.53, 1.14, 1.00},
-        {12, 64, 128, 3, 4.21, 13.31, 0.36, 2.48, 3.1, 0.95, 0.94, 1.02},
+        {10, 128, 128, 2, 0.71, 13.57, 0.45, 5.10, 2.4, 1.53, 1.14, 1.00, 1.15},
+        {12, 64, 128, 3, 4.21, 13.31, 0.36, 2.48, 3.1, 0.95, 0.97, 1.02},
         {16, 128, 256, 1, 5.66, 13.01, 0.65, 2.56, 2.7, 0.82, 0.96, 1.00},
         {18, 256, 256, 1, 15.52, 20.34, 0.67, 0.00, 1.8, 0.81, 0.92, 1.00},
         {19, 128, 320, 1, 10.28, 15.39, 0.73, 1.80, 2.3, 0.75, 1.00, 1.00},
         {20, 64, 192, 1, 3.95, 7.29, 0.83, 2.11, 0.0, 0.00, 1.02, 1.00},
         {21, 128, 192, 1, 5.34, 9.82, 0.67, 3.71, 2.4, 0.89, 1.00, 1.00},
-        {22, 192, 256, 1, 7.80, 16.42, 0.63, 2.46, 2.2, 0.81, 0.92, 1.02},
+        {22, 192, 256, 1, 7.80, 16.42, 0.63, 2.46, 2.2, 0.81, 0.92, 1.02, 1.16},
     };
     const RingChoice c = pick_ring(kFits, sizeof(kFits) / sizeof(kFits[0]), a, cus, ws_limited, split_override);
     return {c.id, c.splits};
@@ -2279,14 +2285,17 @@ W4Plan plan_w4a16(const W8A16Args& a, int cus, bool ws_limited) {
     // within 1 % of the fastest on average, where three rings, split only from
     // K = 4096 on, were 13 % off: 67 x 3328 -> 1664 16 us against 35, 191 x
     // 2816 -> 1280 16 against 30 (128 x 128 tiles two per CU, split four ways);
-    // 192 x 256 tiles 916 x 2560 -> 8704 53 us against 63 in 256 x 256.
+    // 192 x 256 tiles 916 x 2560 -> 8704 53 us against 63 in 256 x 256 (their
+    // splits were 9 % over their fit: 576 x 4608 -> 2324 38 against 32 in 128 x
+    // 128). Against those rules, over 3700 further calls, 0.71 of the time,
+    // slower by more than 3 % on 2 %, by more than 8 % on 0.2 %.
     static constexpr RingFit kFits[] = {
         {4, 256, 128, 1, 4.01, 15.18, 0.72, 7.28, 0.7, 1.24, 1.02, 0.96},
         {5, 128, 128, 1, 1.65, 10.44, 0.77, 5.00, 2.2, 1.32, 0.98, 1.00},
         {10, 128, 128, 2, 0.00, 16.60, 0.56, 5.63, 1.8, 1.78, 1.06, 1.00},
         {16, 128, 256, 1, 0.78, 17.35, 0.73, 5.97, 2.0, 1.40, 0.96, 0.98},
         {18, 256, 256, 1, 8.68, 23.70, 0.73, 3.89, 0.6, 1.25, 1.00, 1.06},
-        {22, 192, 256, 1, 2.84, 21.39, 0.65, 5.12, 2.4, 1.22, 1.00, 0.92},
+        {22, 192, 256, 1, 2.84, 21.39, 0.65, 5.12, 2.4, 1.22, 1.00, 1.00},
     };
     const RingChoice c = pick_ring(kFits, sizeof(kFits) / sizeof(kFits[0]), a, cus, ws_limited, split_override);
     return {c.id, c.splits};
