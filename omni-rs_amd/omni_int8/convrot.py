@@ -232,6 +232,9 @@ class Int8Linear:
         if dims[-1] != self.input:
             # convrot.rs:84 asserts the width
             raise ValueError(f"ConvRot input width {dims[-1]} != {self.input}")
+        if self.scale.numel() != self.output:
+            # the library writes a column per scale
+            raise RuntimeError(f"ConvRot int8 gemm: shapes disagree ({self.scale.numel()} scales, output {self.output})")
         direct = (_lib._host or _lib.host()).convrot_linear(x, self.packed, self.scale, self.zero,
                                                             self.precision is torch.float16)
         if direct is not NotImplemented:

@@ -133,6 +133,16 @@ def _write_layer(path, name, output, input, seed=0, scale_dtype=np.float32, extr
     return t
 
 
+@pytest.mark.parametrize("output", [8, 32])
+def test_layer_refuses_an_output_width_that_its_scales_disagree_with(output):
+    # The library writes one column per scale, the wrapper's buffer has `output`.
+    import torch
+    layer = convrot.Int8Linear(256, output, torch.zeros(16 * 64, dtype=torch.int32), torch.ones(16),
+                               torch.zeros(16, dtype=torch.int32))
+    with pytest.raises(RuntimeError, match="shapes disagree"):
+        layer(torch.zeros((2, 256)))
+
+
 def test_loader_reads_a_layer_written_by_the_safetensors_library(tmp_path):
     import torch
     name = "transformer_blocks.0.attn.to_q"
