@@ -1475,8 +1475,8 @@ int w8a8_split_override() { return knob(Knob::W8A8Splits, 0); }
 // which have neither.
 bool w8a8_pinned() { return w8a8_tile_override() != 0 || w8a8_split_override() > 1; }
 
-// Split K when 256 x 128 tiles fill at most half of the CUs and K >= 4608, or
-// at most an eighth of them and K >= 4096: K split up to 6 ways, at most one
+// The split of K, where plan_w8a8 takes one: 256 x 128 tiles fill at most half
+// of the CUs and K >= 4608, or at most an eighth of them and K >= 4096: K split up to 6 ways, at most one
 // unit per CU, on the 256 x 128 pair ring. The partial sums cost one int32
 // write and read per element and split, so shorter K, or more tiles, do not
 // pay (MI355X, the reference's shapes: 256 x 4096 x 12288 69 -> 29 us, 256 x
@@ -1535,19 +1535,19 @@ struct W8A8Plan {
 //    the tiles fill at most an eighth of the CUs) it runs without regard to
 //    whole; at K = 4608 ... 8191 where it is under 0.8 of it, since both fits
 //    are that uncertain there;
-//  * the streaming kernels (w8a8_rows_us): up to 64 rows unless split K from K
-//    = 8192 on is under theirs by 3 %, or, from 49 rows on, over 16384 columns
-//    and K > 4096 the weight rows are not whole 128-byte lines (56 rows of
+//  * the streaming kernels (w8a8_rows_us): up to 64 rows unless split K over K
+//    >= 8192 is under 1.03 of theirs or, from 49 rows on, over 16384 columns
+//    and K > 4096, the weight rows are not whole 128-byte lines (56 rows of
 //    10048 x 16832 80 us against 69, of 4288 x 17100 37.8 against 35.3; 9472 x
 //    16896 57 against 62); more rows where they are under split K and 0.95 of
 //    whole.
 // Against the choice without the streaming kernels and splits from 8192 on
 // only, 5500 drawn calls (K 1024 ... 14336, N 1024 ... 18944) take 0.46 of the
 // time at 17 to 64 rows, 0.62 at 65 to 256, 0.82 at 257 to 1024 and 0.97 above;
-// 1 % of them are slower by more than 3 %, the worst by 16 %. Streaming all up to 64 rows and
-// comparing tiles with a split fitted to fewer rows was slower on 5 % of 49
-// to 64 rows, by up to half (54 of 12736 x 8512 64 us against 42), and above
-// 1024 rows by up to 1.7 (2049 of 4672 x 1728 62 against 36).
+// 1 % of them are slower by more than 3 %, the worst by 16 %. Streaming all up
+// to 64 rows, and comparing tiles with a split fitted to fewer rows, was slower
+// on 5 % of 49 to 64 rows, by up to half (54 of 12736 x 8512 64 us against 42),
+// and above 1024 rows by up to 1.7 times (2049 of 4672 x 1728 62 against 36).
 double split_us(const W8A8Args& a, int64_t tiles, int splits) {
     const double K = (double)a.width, rows = (double)a.rows, columns = (double)a.columns;
     return 7.76 + 4.52e-3 * K / splits + 1.41e-6 * splits * rows * columns + 7e-8 * K * columns +
