@@ -233,7 +233,7 @@ int omni_convrot_linear(const void* x, int x_dtype, int64_t rows, int64_t width,
  * bias f16 [columns] or NULL, out f16 [rows][columns]. width % 16 == 0.
  * One or two rows (three and four on some shapes) run the HBM-bound GEMV, up
  * to 64 rows kernels that stream the weights past MFMA, more rows (and from
- * 33 on, large matrices) the fp16-MFMA GEMM. */
+ * 17 on, some large matrices) the fp16-MFMA GEMM. */
 int omni_w8a16_gemm(const uint16_t* x, const int8_t* w, const uint16_t* scale,
                     const uint16_t* bias, int64_t rows, int64_t columns, int64_t width,
                     uint16_t* out, void* stream);

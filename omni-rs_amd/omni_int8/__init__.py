@@ -211,8 +211,9 @@ def w8a16_linear(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor,
     """Weight-only int8 linear: f16(scale[n] * sum_k x[m,k] * w[n,k] + bias[n]).
 
     x f16 [rows, width] (leading dims are flattened), w int8 [columns, width],
-    scale/bias f16 [columns] -> f16 [..., columns]. Decode shapes (rows <= 4)
-    run the HBM-bound GEMV, larger ones the fp16-MFMA GEMM."""
+    scale/bias f16 [columns] -> f16 [..., columns]. One or two rows run the
+    HBM-bound GEMV, up to 64 mostly a kernel that streams the weights past MFMA,
+    more the fp16-MFMA GEMM."""
     direct = (_lib._host or _lib.host()).w8a16_linear(x, w, scale, bias)
     if direct is not NotImplemented:
         return direct
